@@ -1938,6 +1938,40 @@ bool ft_forward_block_ok(int mode, bool f16_table, uint32_t ft_out, uint32_t pie
     return false;
 }
 
+// The LDS-resident gather stages the whole table once whatever the batch; the
+// row gather reads only the rows in use, each as often as it occurs.  The
+// line is therefore drawn over the occurrences per table row,
+// 2 * batch * max_active / cols.  Below it the row gather (and the row-major
+// table, which the fold writes faster, and key pass without slot offsets) is
+// the faster one.  Measured as prep + forward + fold of a step, staged / rows,
+// in us (halfka-hm-merged 73305 rows, halfkp 125388 rows):
+//   occurrences   f32 1536   f32 768    f32 512    f32 384    f32 256
+//       4.5       593 / 485  324 / 270  237 / 190  197 / 161  149 / 122
+//       8.9       645 / 588  347 / 313
+//      17.9       734 / 762  393 / 395  289 / 280  278 / 253  207 / 175
+//      35.8       856 / 1051 458 / 539  335 / 378  350 / 342  265 / 218
+//     143                               751 / 976  809 / 955  659 / 536
+//   occurrences   f16 1536   f16 768    f16 512    f16 256
+//      17.9       536 / 510  306 / 306  224 / 193  181 / 162
+//      35.8       634 / 668  356 / 409  269 / 248  219 / 210
+//      71.5       856 / 967  473 / 615  358 / 356  319 / 311
+//     143                    705 / 1002 539 / 572  550 / 513
+//   occurrences   Simple 256 Simple 512 Simple 1024 (f32, concat)
+//       2.6       202 / 134  374 / 257  759 / 534
+//      20.9       277 / 244  480 / 464  926 / 959
+//      41.8       346 / 351  596 / 671  1176 / 1341
+bool ft_forward_block_pays(int mode, bool f16_table, uint32_t ft_out, uint32_t cols, uint32_t max_active,
+                           uint32_t batch) {
+    uint64_t line;  // occurrences per table row
+    if (mode == kConcat) {
+        line = ft_out <= 256 ? 40 : 20;
+    } else {
+        if (ft_out <= 256) return false;
+        line = f16_table ? (ft_out <= 512 ? 80 : 20) : (ft_out < 768 ? 20 : 16);
+    }
+    return 2ull * batch * max_active >= line * cols;
+}
+
 int32_t launch_ft_forward(const FtForwardArgs& a, hipStream_t stream) {
     TATARA_REQUIRE(a.max_active <= (uint32_t)kMaxActive, "max_active must be <= 64");
     TATARA_REQUIRE(a.ft_out % 8 == 0, "ft_out must be a multiple of 8");

@@ -56,6 +56,10 @@ struct FtForwardArgs {
 // Whether the LDS-resident forward serves this shape (mode, table type,
 // ft_out, piece_inputs, max_active); otherwise the row gather runs.
 bool ft_forward_block_ok(int mode, bool f16_table, uint32_t ft_out, uint32_t piece_inputs, uint32_t max_active);
+// Whether it is also the faster form for batches of `batch` positions (the
+// line and the measurements on both sides of it: the definition).
+bool ft_forward_block_pays(int mode, bool f16_table, uint32_t ft_out, uint32_t cols, uint32_t max_active,
+                           uint32_t batch);
 // Slots per row of FtForwardArgs::slot_off (max_active rounded up to 40 or 48;
 // the padding holds the zero row's offset).
 uint32_t ft_block_slot_stride(uint32_t max_active);

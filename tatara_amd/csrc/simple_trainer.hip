@@ -158,7 +158,8 @@ class SimpleTrainer final : public TrainerBase {
             (st = arena.alloc(&sched_count, 2 * n_king_bins)))
             return st;
         if (factorized && n_king_bins == ceil_div(ft_in, pi) &&
-            ft_forward_block_ok(2, false, ft_out, pi, max_active)) {
+            ft_forward_block_ok(2, false, ft_out, pi, max_active) &&
+            ft_forward_block_pays(2, false, ft_out, ft_in, max_active, max_b)) {
             if ((st = arena.alloc(&fb_off, 2 * B * ft_block_slot_stride(max_active), false)) || (st = arena.alloc(&fb_bad, 2 * B, false)))
                 return st;
         }

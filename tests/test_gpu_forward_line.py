@@ -1,0 +1,71 @@
+"""The FT forward on both sides of the line between the LDS-resident gather and
+the row gather (GPU): the oracle's sums bit for bit, whichever form a trainer
+takes for its batch capacity.
+
+The line is drawn over 2 * max_batch * max_active / table rows, so each shape
+comes with a capacity just below it and one on it, with a row whose features
+lie in two king blocks, king blocks of the largest width held in LDS and
+rows padded to 40 and to 48 slots.
+"""
+import numpy as np
+import pytest
+
+from oracle import layerstack as ols
+from oracle import simple as osi
+from tatara_amd.synthetic import small_spec, structured_batch
+from tatara_amd.trainer import Batch, LayerStackConfig, LayerStackTrainer, Sigmoid, SimpleConfig, SimpleTrainer, Wrm
+
+pytestmark = pytest.mark.gpu
+
+SIGMOID = {"kind": "sigmoid", "scale": 1.0 / 290.0}
+WRM = {"kind": "wrm", "nnue2score": 600.0, "in_scaling": 340.0, "in_offset": 270.0, "target_offset": 270.0,
+       "target_scaling": 380.0, "pow_exp": 2.0, "qp_asymmetry": 0.0, "w1": 0.0, "w2": 0.5}
+
+
+def a_batch(b, spec, seed):
+    batch, bucket = structured_batch(b, spec, num_buckets=8, seed=seed, nnz_min=spec["max_active"] - 10)
+    stm = batch.stm_indices.copy()
+    pi, kb = spec["piece_inputs"], spec["king_buckets"]
+    stm[9, 1] = (int(stm[9, 0]) // pi + 1) % kb * pi + 5  # a feature of another king block
+    return Batch(stm, batch.nstm_indices, batch.nnz, batch.score, batch.wdl), bucket
+
+
+# (king blocks, pieces, slots, columns, occurrences per table row on the line)
+@pytest.mark.parametrize("mixed,kb,pi,ma,ft_out,line",
+                         [(False, 10, 64, 40, 512, 20), (False, 10, 64, 44, 640, 20), (False, 10, 64, 38, 768, 16),
+                          (False, 2, 1791, 40, 384, 20), (True, 10, 64, 40, 640, 20), (True, 10, 64, 44, 512, 80)])
+def test_layerstack_forward_on_both_sides(gpu, mixed, kb, pi, ma, ft_out, line):
+    spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
+    sh = ols.LsShape(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, l1=16, l2=32, nb=8)
+    on = -(-line * kb * pi // (2 * ma * 16)) * 16
+    prec = ols.Precision.all_optim() if mixed else ols.FP32
+    for b in (on - 16, on):
+        cfg = LayerStackConfig(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, num_buckets=8,
+                               max_batch=b)
+        batch, bucket = a_batch(b, spec, b)
+        st = ols.default_init(sh)
+        with LayerStackTrainer(cfg.all_optim() if mixed else cfg) as t:
+            _, net = t.validate_step(batch, bucket, 0.0, Sigmoid())
+            a, _ = ols.forward(sh, st, dict(stm=batch.stm_indices, nstm=batch.nstm_indices, nnz=batch.nnz,
+                                            bucket=bucket, score=batch.score, wdl=batch.wdl), 0.0, SIGMOID, prec)
+            for name, key in (("ft_stm_out", "ft_stm"), ("ft_nstm_out", "ft_nstm"), ("combined", "combined")):
+                assert np.array_equal(t.activation(name, b * ft_out), a[key]), (b, name)
+            assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
+
+
+@pytest.mark.parametrize("kb,pi,ma,ft_out,line", [(10, 64, 44, 256, 40), (10, 64, 38, 512, 20), (2, 1791, 40, 128, 40)])
+def test_simple_forward_on_both_sides(gpu, kb, pi, ma, ft_out, line):
+    spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
+    sh = osi.SimpleShape(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, l1=32, l2=32)
+    on = -(-line * kb * pi // (2 * ma))
+    for b in (on - 1, on):
+        batch, _ = a_batch(b, spec, b)
+        st = osi.default_init(sh)
+        with SimpleTrainer(SimpleConfig(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out,
+                                        max_batch=b)) as t:
+            _, net = t.validate_step(batch, 0.0, Wrm())
+            a, _ = osi.forward(sh, st, dict(stm=batch.stm_indices, nstm=batch.nstm_indices, nnz=batch.nnz,
+                                            score=batch.score, wdl=batch.wdl), 0.0, WRM)
+            for name, key, n in (("ft_stm_out", "ft_stm", 1), ("ft_nstm_out", "ft_nstm", 1), ("combined", "combined", 2)):
+                assert np.array_equal(t.activation(name, n * b * ft_out), a[key]), (b, name)
+            assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
