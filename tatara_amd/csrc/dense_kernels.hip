@@ -18,6 +18,8 @@
 // bit-reproducible run to run (no float atomics anywhere).
 #include "dense_kernels.hpp"
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "ft_kernels.hpp"
 
@@ -680,22 +682,28 @@ __global__ __launch_bounds__(256) void ls_l1_wgrad_kernel(LsDenseArgs a) {
 // dcombined[c] = sum_o dl1[o] * l1_w[g][o][c]  +  sum_o dl1[o] * l1s_w[c][o]
 // (the reference's two input-gradient kernels, added as in
 // ft_post_perspective_grad_fused), then the pairwise CReLU gradient into dft
-// (native_kernels.cu:2260-2302).  Grid (column block, row block): a lane owns
-// its columns of the combined output over kPostTiles sorted tiles (the L1
-// gradient row is wave-uniform, the weights stay in registers) and writes
-// its ft_b gradient partials per perspective for that row block.  The f16
+// (native_kernels.cu:2260-2302).  Grid (column block, row block): a wave owns
+// 64 columns of the combined output over post_tiles sorted tiles and writes
+// their ft_b gradient partials per perspective for that row block.  The f16
 // variant reads f16 raw sums and writes the f16 dft, scaled by dft_scale and
 // clamped to +-65504 with a count of every clamp
 // (ft_post_perspective_grad_fused_fp16, native_kernels.cu:2304-2352); the
-// ft_b gradient stays unscaled f32.  For the f32 dft, two columns per lane
-// with rows loaded four at a time measured 5% faster than one column per
-// lane with all 16 rows loaded ahead (0.555 against 0.586 ms for the whole
-// dense backward at ft_out 1536, b 65536), and faster than four columns per
-// lane (193 VGPRs) or one workgroup per full row; for the f16 dft the
-// one-column form stays faster (0.44 against 0.48 ms per launch).  The two
-// 16-term input-gradient sums use
-// fused multiply-adds (these layers are checked within tolerance, and their
-// reference GPU kernels contract too).
+// ft_b gradient stays unscaled f32.
+//
+// The two input gradients are [16 rows][L1] x [L1][64 columns] products per
+// tile on the matrix cores (f32 operands and sums, o ascending).  MFMA operand
+// layout (16x16x4 f32): lane l supplies A[l%16][l/16] and B[l/16][l%16];
+// element r of the result is D[4*(l/16)+r][l%16].  Column group g's column
+// l%16 is the wave's column 4 * (l%16) + g, so a lane ends with four rows of
+// four consecutive columns and moves raw sums and dft in 16-byte (f16:
+// 8-byte) pieces.
+// With the sums as per-column FMAs (32 an element, plus the dl1 broadcasts)
+// the kernel was bound by vector issue in f16.  ft_out 1536, b 65536: f16 273
+// -> 193 us (0.8 GB, 4.2 TB/s), f32 324 -> 324 (1.6 GB, 5.0 TB/s: memory);
+// ft_out 512, l1 32, b 2048: 25 -> 15 us.  The weights wait in LDS (each lane
+// reads back what it wrote, so nothing is synchronised): in registers they
+// cost a wave per SIMD.  The next tile's raw sums loaded ahead measured
+// slower (255 us f16): 32 more registers, one wave per SIMD less.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float clamp_f16_range(float v, uint32_t& clamps) {
     if (v > 65504.0f) {
@@ -709,205 +717,147 @@ __device__ __forceinline__ float clamp_f16_range(float v, uint32_t& clamps) {
     return v;
 }
 
-// Each lane owns CPL consecutive combined columns c..c+CPL-1 (all on one
-// perspective's half); a 128-lane block covers 128 * CPL columns
-// (ft_out % (128 * CPL) == 0).  A tile's rows are taken in groups of RB, an
-// even number of groups per tile.  A tile's row ids, dl1 rows and bin are
-// loaded one tile ahead (lane r holds row r's id, lane i float4 i of the
-// dl1 rows; readlane hands each lane a row's values, which are the same for
-// every lane), and each group's raw-sum pairs are loaded while the group
-// before it is computed (two register sets; the loads are unconditional,
-// from row 0 where a row is padding, so the wait before a group counts only
-// the loads issued after it).  H16: f16 raw sums and dft.
-template <int L1, int CPL, int RB, bool H16>
-__global__ __launch_bounds__(128) void ls_l1_input_post_c_kernel(LsDenseArgs a) {
-    static_assert(16 % RB == 0 && (16 / RB) % 2 == 0, "an even number of RB-row groups per tile");
-    constexpr int G = 16 / RB;
-    constexpr int DL = 16 * L1 / 4;          // float4 of a tile's dl1 rows
-    constexpr int NDL = (DL + 63) / 64;      // of them per lane
-    static_assert(L1 % 4 == 0, "whole float4 of dl1 per row");
+template <int L1, bool H16>
+__global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, uint32_t post_tiles) {
+    constexpr int KC = L1 / 4;  // MFMAs per column group and gradient
+    static_assert(L1 % 4 == 0, "whole MFMAs");
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    using Raw = typename std::conditional<H16, h4, floatx4>::type;
+    // a lane's own weights of the current bucket: [bucket, shared][k][lane]
+    __shared__ floatx4 s_w[2][KC][128];
     const uint32_t ft_out = a.ft_out, half = ft_out / 2;
     const uint64_t batch = a.batch;
-    const uint32_t c = (blockIdx.x * 128 + threadIdx.x) * CPL;
-    if (c >= ft_out) return;
-    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t tid = threadIdx.x, lane = tid % 64, i = lane % 16, q = lane / 16;
+    // ft_out % 128 == 0: the wave's 64 columns lie in one perspective's half
+    const uint32_t c = (blockIdx.x * 2 + tid / 64) * 64 + 4 * i;
     const uint32_t persp = c < half ? 0 : 1;
     const uint32_t p = c - persp * half;
-    const _Float16* ft16 = reinterpret_cast<const _Float16*>(persp ? a.ft_nstm16 : a.ft_stm16);
-    const float* ft32 = persp ? a.ft_nstm : a.ft_stm;
+    const Raw* raw = reinterpret_cast<const Raw*>(
+        H16 ? static_cast<const void*>(persp ? a.ft_nstm16 : a.ft_stm16)
+            : static_cast<const void*>(persp ? a.ft_nstm : a.ft_stm));
+    // chunk-major dft: p and p + half are multiples of four, so a lane's run
+    // lies in one chunk
     const uint64_t cstride = 2 * batch * kDftChunk;
     const uint64_t off_a = (uint64_t)(p / kDftChunk) * cstride + persp * batch * kDftChunk + p % kDftChunk;
     const uint64_t off_b =
         (uint64_t)((p + half) / kDftChunk) * cstride + persp * batch * kDftChunk + (p + half) % kDftChunk;
-    float ws[CPL][L1];
+    Raw* dft = reinterpret_cast<Raw*>(H16 ? static_cast<void*>(a.dft16) : static_cast<void*>(a.dft));
+    const floatx4 ba = *reinterpret_cast<const floatx4*>(a.ft_b + p);
+    const floatx4 bb = *reinterpret_cast<const floatx4*>(a.ft_b + p + half);
 #pragma unroll
-    for (int j = 0; j < CPL; ++j)
+    for (int k = 0; k < KC; ++k) {
+        floatx4 v;
 #pragma unroll
-        for (int o = 0; o < L1; ++o) ws[j][o] = a.l1s_w[(uint64_t)(c + j) * L1 + o];
-    float ba[CPL], bb[CPL];
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-        ba[j] = a.ft_b[p + j];
-        bb[j] = a.ft_b[p + half + j];
+        for (int g = 0; g < 4; ++g) v[g] = a.l1s_w[(uint64_t)(c + g) * L1 + 4 * k + q];
+        s_w[1][k][tid] = v;
     }
-    float w1[CPL][L1];
     int32_t cur_bin = -2;
-    bool bvalid = false;
-    float acc_a[CPL] = {}, acc_b[CPL] = {};
+    floatx4 acc_a = {0.f, 0.f, 0.f, 0.f}, acc_b = {0.f, 0.f, 0.f, 0.f};
     uint32_t clamps = 0;
-    const uint32_t tile0 = blockIdx.y * kPostTiles;
+    const uint32_t tile0 = blockIdx.y * post_tiles;
     const uint32_t tiles_total = (uint32_t)(a.padded_b / 16);
-    const uint32_t n_tiles = tile0 < tiles_total ? min((uint32_t)kPostTiles, tiles_total - tile0) : 0u;
-    auto tile_perm = [&](uint32_t tile) -> int32_t { return a.perm[(uint64_t)tile * 16 + (lane & 15u)]; };
-    struct Dl1 {
-        float4 v[NDL];
+    const uint32_t n_tiles = tile0 < tiles_total ? min(post_tiles, tiles_total - tile0) : 0u;
+    if (n_tiles == 0) return;  // the grid covers whole row blocks only
+    struct Tile {
+        int4 rows;    // original rows of 4q .. 4q+3
+        float d[KC];  // dl1 of row i, k = 4c + q
+        int32_t bin;
     };
-    // float4 f of the tile's dl1 rows is element f / 64 of lane f % 64
-    auto tile_dl1 = [&](uint32_t tile) -> Dl1 {
-        Dl1 d;
-        const float4* src = reinterpret_cast<const float4*>(a.dl1_sorted + (uint64_t)tile * 16 * L1);
+    auto load_tile = [&](uint32_t tile) -> Tile {
+        Tile t;
+        t.rows = *reinterpret_cast<const int4*>(a.perm + (uint64_t)tile * 16 + 4 * q);
 #pragma unroll
-        for (int k = 0; k < NDL; ++k) d.v[k] = src[(64 * k + lane) % DL];
-        return d;
+        for (int k = 0; k < KC; ++k) t.d[k] = a.dl1_sorted[((uint64_t)tile * 16 + i) * L1 + 4 * k + q];
+        t.bin = scalar_load(a.sorted_bin + (uint64_t)tile * 16);
+        return t;
     };
-    auto bcast_i = [](int32_t v, int l) -> int32_t { return __builtin_amdgcn_readlane(v, l); };
-    auto bcast_f = [](float v, int l) -> float {
-        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-    };
-    float xr[2][RB][CPL], yr[2][RB][CPL];
-    // group G0's raw-sum pairs (row ids from PERMV) into register set BUF
-#define TATARA_POST_LOAD(BUF, PERMV, G0)                                                      \
-    _Pragma("unroll") for (int r = 0; r < RB; ++r) {                                         \
-        const int32_t o_ = bcast_i((PERMV), (G0) * RB + r);                                  \
-        const uint64_t base = (uint64_t)(o_ >= 0 ? o_ : 0) * ft_out + p;                      \
-        if constexpr (CPL == 1) {                                                             \
-            xr[BUF][r][0] = H16 ? (float)ft16[base] : ft32[base];                             \
-            yr[BUF][r][0] = H16 ? (float)ft16[base + half] : ft32[base + half];               \
-        } else if constexpr (H16) {                                                           \
-            typedef _Float16 h2 __attribute__((ext_vector_type(2)));                          \
-            const h2 x_ = *reinterpret_cast<const h2*>(ft16 + base);                          \
-            const h2 y_ = *reinterpret_cast<const h2*>(ft16 + base + half);                   \
-            xr[BUF][r][0] = (float)x_.x;                                                      \
-            xr[BUF][r][1] = (float)x_.y;                                                      \
-            yr[BUF][r][0] = (float)y_.x;                                                      \
-            yr[BUF][r][1] = (float)y_.y;                                                      \
-        } else {                                                                              \
-            const float2 x_ = *reinterpret_cast<const float2*>(ft32 + base);                  \
-            const float2 y_ = *reinterpret_cast<const float2*>(ft32 + base + half);           \
-            xr[BUF][r][0] = x_.x;                                                             \
-            xr[BUF][r][1] = x_.y;                                                             \
-            yr[BUF][r][0] = y_.x;                                                             \
-            yr[BUF][r][1] = y_.y;                                                             \
-        }                                                                                     \
-    }
-    int32_t perm_c = 0, bin_c = -1;
-    Dl1 dl1_c = {};
-    if (n_tiles) {
-        perm_c = tile_perm(tile0);
-        dl1_c = tile_dl1(tile0);
-        bin_c = scalar_load(a.sorted_bin + (uint64_t)tile0 * 16);
-        TATARA_POST_LOAD(0, perm_c, 0)
-    }
+    Tile cur = load_tile(tile0);
     for (uint32_t t = 0; t < n_tiles; ++t) {
-        const uint32_t tile = tile0 + t;
-        const bool has_next = t + 1 < n_tiles;
-        const uint32_t tn = has_next ? tile + 1 : tile;  // the last tile re-reads itself, unused
-        const int32_t perm_n = tile_perm(tn);
-        const Dl1 dl1_n = tile_dl1(tn);
-        const int32_t bin_n = has_next ? scalar_load(a.sorted_bin + (uint64_t)tn * 16) : -1;
-        const int32_t bin = bin_c;  // < 0: a trailing all-padding tile
-        if (bin >= 0 && bin != cur_bin) {
-            cur_bin = bin;
-            bvalid = (uint32_t)bin < a.nb;
+        // the next tile's ids and dl1 (the last tile re-reads itself, unused)
+        const Tile next = load_tile(t + 1 < n_tiles ? tile0 + t + 1 : tile0 + t);
+        if (cur.bin >= 0) {  // else a trailing all-padding tile
+            const int32_t rows[4] = {cur.rows.x, cur.rows.y, cur.rows.z, cur.rows.w};
+            Raw xr[4], yr[4];
 #pragma unroll
-            for (int o = 0; o < L1; ++o) {
-                const uint64_t i = ((uint64_t)bin * L1 + o) * ft_out + c;
-                if constexpr (CPL == 2) {
-                    const float2 w = bvalid ? *reinterpret_cast<const float2*>(a.l1_w + i) : make_float2(0.0f, 0.0f);
-                    w1[0][o] = w.x;
-                    w1[1][o] = w.y;
-                } else {
-                    w1[0][o] = bvalid ? a.l1_w[i] : 0.0f;
+            for (int r = 0; r < 4; ++r) {  // row 0 (always valid) where the row is padding
+                const uint64_t base = (uint64_t)(rows[r] >= 0 ? rows[r] : 0) * ft_out + p;
+                xr[r] = raw[base / 4];
+                yr[r] = raw[(base + half) / 4];
+            }
+            if (cur.bin != cur_bin) {
+                cur_bin = cur.bin;
+                const bool bvalid = (uint32_t)cur_bin < a.nb;
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    const floatx4 wb = *reinterpret_cast<const floatx4*>(
+                        a.l1_w + ((uint64_t)(bvalid ? cur_bin : 0) * L1 + 4 * k + q) * ft_out + c);
+                    s_w[0][k][tid] = bvalid ? wb : floatx4{0.f, 0.f, 0.f, 0.f};
                 }
             }
-        }
+            floatx4 da[4], db[4];  // [column group][row]
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            // the next group's loads first: of this tile, or the next tile's first
-            if (g + 1 < G) {
-                TATARA_POST_LOAD((g + 1) & 1, perm_c, g + 1)
-            } else {
-                TATARA_POST_LOAD(0, perm_n, 0)
+            for (int g = 0; g < 4; ++g) da[g] = db[g] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KC; ++k) {
+                const floatx4 w1 = s_w[0][k][tid], ws = s_w[1][k][tid];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    da[g] = mfma4(cur.d[k], w1[g], da[g]);
+                    db[g] = mfma4(cur.d[k], ws[g], db[g]);
+                }
             }
-            if (bin < 0) continue;
 #pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const int row_in_tile = g * RB + r;
-                const int32_t orig = bcast_i(perm_c, row_in_tile);
-                if (orig < 0) continue;
-                float d[L1];
+            for (int g = 0; g < 4; ++g) da[g] += db[g];
 #pragma unroll
-                for (int o = 0; o < L1; ++o) {
-                    const int e = row_in_tile * L1 + o, f4 = e >> 2;
-                    const float4& v = dl1_c.v[f4 / 64];
-                    const float comp = (e & 3) == 0 ? v.x : (e & 3) == 1 ? v.y : (e & 3) == 2 ? v.z : v.w;
-                    d[o] = bcast_f(comp, f4 % 64);
+            for (int r = 0; r < 4; ++r) {
+                if (rows[r] < 0) continue;
+                floatx4 ga, gb;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float xa = (float)xr[r][g] + ba[g], xb = (float)yr[r][g] + bb[g];
+                    const float dy = da[g][r];
+                    ga[g] = (xa > 0.0f && xa < 1.0f) ? dy * crelu01(xb) * a.ft_post_scale : 0.0f;
+                    gb[g] = (xb > 0.0f && xb < 1.0f) ? dy * crelu01(xa) * a.ft_post_scale : 0.0f;
                 }
-                float ga[CPL], gb[CPL];
-#pragma unroll
-                for (int j = 0; j < CPL; ++j) {
-                    float da = 0.0f;
-                    if (bvalid) {
-#pragma unroll
-                        for (int o = 0; o < L1; ++o) da = __builtin_fmaf(d[o], w1[j][o], da);
-                    }
-                    float db = 0.0f;
-#pragma unroll
-                    for (int o = 0; o < L1; ++o) db = __builtin_fmaf(d[o], ws[j][o], db);
-                    const float dy = da + db;
-                    const float xa = xr[g & 1][r][j] + ba[j], xb = yr[g & 1][r][j] + bb[j];
-                    const float ya = crelu01(xa), yb = crelu01(xb);
-                    ga[j] = (xa > 0.0f && xa < 1.0f) ? dy * yb * a.ft_post_scale : 0.0f;
-                    gb[j] = (xb > 0.0f && xb < 1.0f) ? dy * ya * a.ft_post_scale : 0.0f;
-                    acc_a[j] += ga[j];
-                    acc_b[j] += gb[j];
-                }
-                const uint64_t row = (uint64_t)orig * kDftChunk;
+                acc_a += ga;
+                acc_b += gb;
+                const uint64_t row = (uint64_t)rows[r] * kDftChunk;
                 if constexpr (H16) {
-                    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-                    const float sc = a.dft_scale;
-                    _Float16* d16 = reinterpret_cast<_Float16*>(a.dft16);
-                    if constexpr (CPL == 2) {
-                        h2 va, vb;
-                        va.x = (_Float16)clamp_f16_range(ga[0] * sc, clamps);
-                        va.y = (_Float16)clamp_f16_range(ga[1] * sc, clamps);
-                        vb.x = (_Float16)clamp_f16_range(gb[0] * sc, clamps);
-                        vb.y = (_Float16)clamp_f16_range(gb[1] * sc, clamps);
-                        *reinterpret_cast<h2*>(d16 + off_a + row) = va;
-                        *reinterpret_cast<h2*>(d16 + off_b + row) = vb;
-                    } else {
-                        d16[off_a + row] = (_Float16)clamp_f16_range(ga[0] * sc, clamps);
-                        d16[off_b + row] = (_Float16)clamp_f16_range(gb[0] * sc, clamps);
+                    floatx4 va = ga * a.dft_scale, vb = gb * a.dft_scale;
+                    // one test of the largest magnitude (a NaN is ignored and
+                    // passes, uncounted) keeps the clamps off the usual path
+                    float top = 0.0f;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) top = fmaxf(top, fmaxf(fabsf(va[g]), fabsf(vb[g])));
+                    if (top > 65504.0f) {
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            va[g] = clamp_f16_range(va[g], clamps);
+                            vb[g] = clamp_f16_range(vb[g], clamps);
+                        }
                     }
-                } else if constexpr (CPL == 2) {
-                    *reinterpret_cast<float2*>(a.dft + off_a + row) = make_float2(ga[0], ga[1]);
-                    *reinterpret_cast<float2*>(a.dft + off_b + row) = make_float2(gb[0], gb[1]);
+                    dft[(off_a + row) / 4] = __builtin_convertvector(va, h4);
+                    dft[(off_b + row) / 4] = __builtin_convertvector(vb, h4);
                 } else {
-                    a.dft[off_a + row] = ga[0];
-                    a.dft[off_b + row] = gb[0];
+                    dft[(off_a + row) / 4] = ga;
+                    dft[(off_b + row) / 4] = gb;
                 }
             }
         }
-        perm_c = perm_n;
-        dl1_c = dl1_n;
-        bin_c = bin_n;
+        cur = next;
     }
-#undef TATARA_POST_LOAD
-    float* pp = a.ftb_partial + ((uint64_t)blockIdx.y * 2 + persp) * ft_out;
+    // the four lanes of a column run hold different rows' sums
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-        pp[p + j] = acc_a[j];
-        pp[p + half + j] = acc_b[j];
+    for (int g = 0; g < 4; ++g) {
+        acc_a[g] += __shfl_xor(acc_a[g], 16);
+        acc_b[g] += __shfl_xor(acc_b[g], 16);
+        acc_a[g] += __shfl_xor(acc_a[g], 32);
+        acc_b[g] += __shfl_xor(acc_b[g], 32);
+    }
+    if (q == 0) {
+        float* pp = a.ftb_partial + ((uint64_t)blockIdx.y * 2 + persp) * ft_out;
+        *reinterpret_cast<floatx4*>(pp + p) = acc_a;
+        *reinterpret_cast<floatx4*>(pp + p + half) = acc_b;
     }
     if (H16 && clamps) atomicAdd(a.clamp_counter, (unsigned long long)clamps);
 }
@@ -996,7 +946,11 @@ __global__ __launch_bounds__(256) void ls_dense_finalize_kernel(LsDenseArgs a, G
 }  // namespace
 
 uint32_t ls_tail_workgroups(uint32_t padded_b) { return ceil_div(padded_b, 16); }
-uint32_t ls_post_workgroups(uint32_t padded_b) { return ceil_div(padded_b / 16, kPostTiles); }
+static uint32_t post_tiles(uint32_t padded_b, uint32_t ft_out) { return post_block_tiles(padded_b / 16, ft_out); }
+static uint32_t post_row_blocks(uint32_t padded_b, uint32_t ft_out) {
+    return ceil_div(padded_b / 16, post_tiles(padded_b, ft_out));
+}
+uint32_t ls_post_workgroups(uint32_t padded_b, uint32_t ft_out) { return post_max_blocks(padded_b / 16, ft_out); }
 uint32_t ls_max_chunks(uint32_t padded_b, uint32_t nb) {
     return ceil_div(padded_b / 16, kChunkTiles) + nb + 1;
 }
@@ -1081,26 +1035,18 @@ int32_t launch_ls_l1_weight_grad(const LsDenseArgs& a, hipStream_t stream) {
 int32_t launch_ls_l1_input_post(const LsDenseArgs& a, hipStream_t stream) {
     TATARA_REQUIRE(!a.dft16 || (a.ft_stm16 && a.ft_nstm16 && a.clamp_counter),
                    "an f16 dft needs the f16 raw sums and a clamp counter");
-    const uint32_t rows = ls_post_workgroups(a.padded_b);
+    const uint32_t rows = post_row_blocks(a.padded_b, a.ft_out);
     if (rows == 0) return kOk;
     TATARA_REQUIRE(a.ft_out % 128 == 0, "ft_out must be a multiple of 128");
     TATARA_REQUIRE(a.l1 == 8 || a.l1 == 16 || a.l1 == 32, kLsDenseShapes);
-    // two columns per lane (f32, l1 <= 16) where the 256-column blocks tile
-    // ft_out; l1 = 32 keeps one column per lane (its 64 weights per column
-    // stay in registers)
-    const bool two = !a.dft16 && a.ft_out % 256 == 0 && a.l1 <= 16;
-    const dim3 grid(a.ft_out / (two ? 256 : 128), rows);
-    // f32: two columns per lane, rows four at a time; f16: one column per
-    // lane, all 16 rows of a tile ahead (each measured fastest for its type)
-    auto kernel = a.dft16 ? (a.l1 == 32   ? ls_l1_input_post_c_kernel<32, 1, 8, true>
-                             : a.l1 == 16 ? ls_l1_input_post_c_kernel<16, 1, 8, true>
-                                          : ls_l1_input_post_c_kernel<8, 1, 8, true>)
-                  : two   ? (a.l1 == 16 ? ls_l1_input_post_c_kernel<16, 2, 4, false>
-                                        : ls_l1_input_post_c_kernel<8, 2, 4, false>)
-                          : (a.l1 == 32   ? ls_l1_input_post_c_kernel<32, 1, 4, false>
-                             : a.l1 == 16 ? ls_l1_input_post_c_kernel<16, 1, 4, false>
-                                          : ls_l1_input_post_c_kernel<8, 1, 4, false>);
-    kernel<<<grid, 128, 0, stream>>>(a);
+    const dim3 grid(a.ft_out / 128, rows);
+    auto kernel = a.dft16 ? (a.l1 == 32   ? ls_l1_input_post_kernel<32, true>
+                             : a.l1 == 16 ? ls_l1_input_post_kernel<16, true>
+                                          : ls_l1_input_post_kernel<8, true>)
+                          : (a.l1 == 32   ? ls_l1_input_post_kernel<32, false>
+                             : a.l1 == 16 ? ls_l1_input_post_kernel<16, false>
+                                          : ls_l1_input_post_kernel<8, false>);
+    kernel<<<grid, 128, 0, stream>>>(a, post_tiles(a.padded_b, a.ft_out));
     TATARA_LAUNCHED("ls_l1_input_post");
     return kOk;
 }
@@ -1117,7 +1063,7 @@ int32_t launch_ls_dense_finalize(const LsDenseArgs& a, LsDenseGroup* groups,
     const uint64_t n = gt.start[9];
     const TailDims td{a.l1, a.l2, a.nb};
     const uint32_t n_tail = ls_tail_workgroups(a.padded_b);
-    const uint32_t n_post = ls_post_workgroups(a.padded_b);
+    const uint32_t n_post = post_row_blocks(a.padded_b, a.ft_out);
     // bucket g's tile partials are the rows [tail_seg[g], tail_seg[g + 1])
     reduce_rows(a.tail_partial, n_tail, td.cells(), a.tail_seg, a.nb, a.tail_sum, stream);
     reduce_rows(a.b1s_partial, n_tail, a.l1, nullptr, 1, a.b1s_sum, stream);

@@ -30,10 +30,6 @@ struct SimpleTailDims {
 };
 
 constexpr uint32_t kSimpleChunkRows = 256;   // rows per L1 weight-gradient chunk
-// rows per L1-input/FT-post workgroup: 64 keeps twice the waves of 128 in
-// flight (Simple 256x2-32-32, b = 65536: dense backward 0.145 against
-// 0.187 ms; 32 rows, 0.149 ms plus the larger partial reduction)
-constexpr uint32_t kSimplePostRows = 64;
 
 struct SimpleDenseArgs {
     uint32_t batch, ft_out, l1, l2;
@@ -67,7 +63,8 @@ struct SimpleDenseArgs {
 
 uint32_t simple_tail_workgroups(uint32_t batch);
 uint32_t simple_chunks(uint32_t batch);
-uint32_t simple_post_workgroups(uint32_t batch);
+// row blocks (ft_b partials) of the input-gradient kernel, at most, up to batch
+uint32_t simple_post_workgroups(uint32_t batch, uint32_t ft_out);
 
 // L1 forward (MFMA): l1_pre = combined . l1_w + l1_b.
 int32_t launch_simple_l1_forward(const SimpleDenseArgs& a, hipStream_t stream);

@@ -1,0 +1,55 @@
+"""The dense kernels at the edges of their tiles (GPU): batches of one row tile
+and one more row, waves whose columns end inside the row, buckets without
+rows, and batches large enough that a workgroup takes several tiles.
+One step against the oracle with the one-step bars of the trainer tests."""
+import numpy as np
+import pytest
+
+from oracle import layerstack as ols
+from oracle import simple as osi
+from tatara_amd.trainer import GROUPS, SIMPLE_GROUPS, LayerStackTrainer, Sigmoid, SimpleTrainer
+
+import test_gpu_simple as gs
+import test_gpu_trainer as gt
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ft_out,l1,l2,b", [(32, 8, 16, 1), (96, 16, 32, 17), (160, 32, 64, 33), (96, 32, 32, 255),
+                                            (64, 8, 32, 16), (32, 32, 16, 40000)])
+def test_simple_edges(gpu, ft_out, l1, l2, b):
+    sh, cfg = gs.make(ft_out=ft_out, l1=l1, l2=l2, optimizer="adamw", b=b)
+    batch = gs.batch_for(b, b)
+    st = osi.default_init(sh)
+    with SimpleTrainer(cfg) as t:
+        t.train_step(batch, 1e-3, 0.25, gs.WRM290)
+        _, a, g = osi.train_step(sh, st, gs.as_dict(batch), osi.OptConfig(), 1e-3, 0.25, gs.loss_dict(gs.WRM290), 1)
+        gs.close(t.activation("l1_pre", b * l1), a["l1_pre"], 1e-5, atol=1e-6, what="l1_pre")
+        gs.close(t.activation("net_output", b), a["net"], 1e-5, atol=1e-6, what="net_output")
+        for name in ("dft_stm", "dft_nstm"):
+            top = max(np.abs(a[name]).max(), 1e-30)
+            gs.close(t.activation(name, b * ft_out), a[name], 1e-4, atol=1e-5 * top, what=name)
+        for name in SIMPLE_GROUPS:
+            gs.close(t.get(name, "grad"), g[name], 1e-4, atol_frac=1e-5, what=f"grad {name}")
+
+
+@pytest.mark.parametrize("ft_out,l1,l2,b,factorize", [(128, 8, 16, 16, True), (384, 16, 32, 48, True),
+                                                      (128, 32, 64, 272, False), (640, 32, 16, 1040, True),
+                                                      (128, 16, 64, 34000, False)])
+def test_layerstack_edges(gpu, ft_out, l1, l2, b, factorize):
+    sh, cfg = gt.make(ft_out=ft_out, l1=l1, l2=l2, b=b, factorize=factorize)
+    batch, bucket = gt.batch_for(b, b, sh.nb)
+    bucket[bucket == 2] = 5  # a bucket without rows
+    st = ols.default_init(sh)
+    loss = Sigmoid()
+    with LayerStackTrainer(cfg) as t:
+        t.train_step(batch, bucket, 8.75e-4, 0.25, loss)
+        _, a, g = ols.train_step(sh, st, gt.as_dict(batch, bucket), ols.OptConfig(), 8.75e-4, 0.25,
+                                 gt.loss_dict(loss), 1)
+        gt.close(t.activation("l1_total", b * l1), a["l1_total"], 1e-5, atol=1e-6, what="l1_total")
+        gt.close(t.activation("net_output", b), a["net"], 1e-5, atol=1e-6, what="net_output")
+        for name in ("dft_stm", "dft_nstm"):
+            top = max(np.abs(a[name]).max(), 1e-30)
+            gt.close(t.activation(name, b * ft_out), a[name], 1e-4, atol=1e-5 * top, what=name)
+        for name in GROUPS:
+            gt.close(t.get(name, "grad"), g[name], 1e-4, atol_frac=1e-5, what=f"grad {name}")
