@@ -303,12 +303,20 @@ __global__ __launch_bounds__(256) void sum_partials_f64_kernel(const double* __r
 // ---------------------------------------------------------------------------
 // Tail: one 64-lane workgroup per sorted 16-row tile (one bucket, the tile's
 // rows being bucket-sorted and 16-aligned).  Lane l serves row r = l % 16 with
-// quarter q = l / 16: its eight L2 outputs o = 8q..8q+7 in the forward, the
+// quarter q = l / 16: its L2/4 consecutive L2 outputs in the forward, the
 // L2 inputs k = q, q+4, .. in the backward, the L1 outputs k = q, q+4, .. of
-// the L1-tail gradient.  The bucket's L2/L3 weights are staged in LDS.  Every
+// the L1-tail gradient.  The tile's L1 outputs, activations and gradients and
+// the bucket's L2/L3 weights are in LDS, the L2 weights transposed so that a
+// lane reads four outputs' weights at once.  Every
 // per-row sum keeps the reference order (k ascending for L2, o ascending for
 // L3 and for the L2 input gradient); the gradient partials are per tile, rows
-// in order, and are reduced per bucket over the bucket's tiles.
+// in order (the L2 weights' as f32 MFMAs over the tile's rows), and are
+// reduced per bucket over the bucket's tiles.
+//
+// Bound by its chain of LDS round trips.  The L1 outputs as per-lane arrays
+// indexed by lane went to scratch memory at l1 = 32, and every cell of the L2
+// weight gradient read 32 LDS words: l1 32, l2 64, b 2048 88 -> 31 us;
+// l1 16, l2 32, b 65536 70 -> 38 us; l1 8, l2 32, b 16384 22 -> 15 us.
 // ---------------------------------------------------------------------------
 template <int L1, int L2>
 __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t train) {
@@ -317,12 +325,16 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
     constexpr int OQ = L2 / 4;             // L2 outputs per lane
     constexpr int KQ = (LIN + 3) / 4;      // L2 inputs per lane (backward)
     constexpr int JQ = L1 / 4;             // L1 outputs per lane (backward)
-    static_assert(L2 % 4 == 0 && L1 % 4 == 0, "quarters");
-    __shared__ float sW2[L2 * LIN];
+    constexpr int WS = L2 + 4;             // row stride of the transposed weights: 16-byte rows, spread banks
+    constexpr int KT = (LIN + 15) / 16;    // 16-input tiles of the L2 weight gradient
+    constexpr int IS = 16 * KT + 1;        // row stride of the L2 inputs (zero past LIN)
+    static_assert(L2 % 16 == 0 && L1 % 4 == 0, "quarters of whole float4, whole MFMA tiles");
+    __shared__ __align__(16) float sW2[LIN * WS];  // [k][o]
     __shared__ float sB2[L2], sW3[L2];
-    __shared__ float s_l2in[16][LIN + 1];
+    __shared__ float s_l1t[16][L1 + 1];
+    __shared__ float s_l2in[16][IS];
     __shared__ float s_l2a[16][L2 + 1];
-    __shared__ float s_dl2o[16][L2 + 1];
+    __shared__ __align__(16) float s_dl2o[16][WS];
     __shared__ float s_dl2pre[16][LIN + 1];
     __shared__ float s_dl1[16][L1 + 1];
     __shared__ float s_dy[16];
@@ -338,58 +350,75 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
     const int32_t bin = orig0 >= 0 ? a.sorted_bin[tile * 16] : -1;
     const bool bvalid = bin >= 0 && (uint32_t)bin < a.nb;
     const int g = bvalid ? bin : 0;
+    const int32_t orig = a.perm[row];
+    const bool real = orig >= 0;
+    if (q == 0) s_real[r] = real ? 1 : 0;
     if (bvalid) {
         const float* W2 = a.l2_w + (uint64_t)g * L2 * LIN;
-        for (uint32_t i = lane; i < (uint32_t)(L2 * LIN); i += 64) sW2[i] = W2[i];
+        // 16-byte loads (a bucket's weights are a multiple of 16 floats), four
+        // in flight: one at a time this loop was most of the kernel
+        constexpr uint32_t N4 = L2 * LIN / 4, U = 4;
+        for (uint32_t i0 = lane; i0 < N4; i0 += 64 * U) {
+            float4 v[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const uint32_t i = i0 + 64 * u;
+                v[u] = reinterpret_cast<const float4*>(W2)[i < N4 ? i : N4 - 1];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                if (i0 + 64 * u >= N4) break;
+                const uint32_t e = 4 * (i0 + 64 * u);
+                const float c[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) sW2[(e + j) % LIN * WS + (e + j) / LIN] = c[j];
+            }
+        }
         if (lane < (uint32_t)L2) {
             sB2[lane] = a.l2_b[g * L2 + lane];
             sW3[lane] = a.l3_w[g * L2 + lane];
         }
     }
     const float b3 = bvalid ? a.l3_b[g] : 0.0f;
-    const int32_t orig = a.perm[row];
-    const bool real = orig >= 0;
-
-    float l1t[L1], l2pre[LIN], l2in[LIN];
-    float skip = 0.0f;
-    if (real) {
-        const float* l1v = a.l1_sorted + row * 2 * L1;
+    __syncthreads();  // s_real
+    // bucket + shared L1 outputs, and what L2 reads of them; zero for padding
+    const float* l1v = a.l1_sorted + tile * 16 * 2 * L1;
 #pragma unroll
-        for (int o = 0; o < L1; ++o) l1t[o] = l1v[o] + l1v[L1 + o];  // elementwise_add
-        skip = l1t[L1 - 1];                                          // slice_extract_2d
-#pragma unroll
-        for (int k = 0; k < LE; ++k) {
-            const float mk = l1t[k];
-            l2pre[k] = mk * mk * a.l1_sqr_scale;  // abs_pow2_scale_fwd
-            l2pre[LE + k] = mk;                   // concat_l1sqr_main_fwd
+    for (uint32_t i = lane; i < 16u * L1; i += 64) {
+        const uint32_t rr = i / L1, o = i % L1;
+        const bool ok = s_real[rr] != 0;
+        const float x = l1v[rr * 2 * L1 + o], y = l1v[rr * 2 * L1 + L1 + o];
+        const float t = ok ? x + y : 0.0f;  // elementwise_add
+        s_l1t[rr][o] = t;
+        if (o < (uint32_t)LE) {
+            s_l2in[rr][o] = crelu01(t * t * a.l1_sqr_scale);  // abs_pow2_scale_fwd
+            s_l2in[rr][LE + o] = crelu01(t);                  // concat_l1sqr_main_fwd
         }
-#pragma unroll
-        for (int k = 0; k < LIN; ++k) l2in[k] = crelu01(l2pre[k]);
-    } else {
-#pragma unroll
-        for (int o = 0; o < L1; ++o) l1t[o] = 0.0f;
-#pragma unroll
-        for (int k = 0; k < LIN; ++k) l2pre[k] = l2in[k] = 0.0f;
     }
-    __syncthreads();  // staged weights visible
+    if (lane < 16)
+        for (int k = LIN; k < 16 * KT; ++k) s_l2in[lane][k] = 0.0f;
+    __syncthreads();
     // L2 (dense_mm_fwd_bucket: the sum starts at the bias, k ascending) + CReLU
     float l2o[OQ];
 #pragma unroll
-    for (int j = 0; j < OQ; ++j) {
-        const int o = OQ * q + j;
-        float acc = bvalid ? sB2[o] : 0.0f;
-        if (bvalid) {
+    for (int j = 0; j < OQ; ++j) l2o[j] = bvalid ? sB2[OQ * q + j] : 0.0f;
+    if (bvalid) {
+#pragma unroll 4
+        for (int k = 0; k < LIN; ++k) {
+            const float x = s_l2in[r][k];
+            const float4* w = reinterpret_cast<const float4*>(sW2 + k * WS + OQ * q);
 #pragma unroll
-            for (int k = 0; k < LIN; ++k) acc += l2in[k] * sW2[o * LIN + k];
+            for (int j = 0; j < OQ; j += 4) {
+                const float4 w4 = w[j / 4];
+                l2o[j + 0] += x * w4.x;
+                l2o[j + 1] += x * w4.y;
+                l2o[j + 2] += x * w4.z;
+                l2o[j + 3] += x * w4.w;
+            }
         }
-        l2o[j] = bvalid ? acc : 0.0f;
-        s_l2a[r][o] = real ? crelu01(l2o[j]) : 0.0f;
     }
-    if (q == 0) {
 #pragma unroll
-        for (int k = 0; k < LIN; ++k) s_l2in[r][k] = l2in[k];
-        s_real[r] = real ? 1 : 0;
-    }
+    for (int j = 0; j < OQ; ++j) s_l2a[r][OQ * q + j] = real ? crelu01(l2o[j]) : 0.0f;
     __syncthreads();
     if (q == 0) {
         // L3 (o ascending from the bias), net = l3 + skip, loss
@@ -402,7 +431,7 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
 #pragma unroll
                 for (int o = 0; o < L2; ++o) l3 += s_l2a[r][o] * sW3[o];
             }
-            const float net = l3 + skip;
+            const float net = l3 + s_l1t[r][LE];  // slice_extract_2d: the skip output
             a.net_output[orig] = net;
             loss_c = position_loss(net, a.score[orig], a.wdl[orig], a.wdl_lambda, a.loss, a.per_pos_norm,
                                    a.weight_sum, a.batch, dy);
@@ -430,16 +459,31 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
     }
     __syncthreads();
     // L2 input gradient for this lane's inputs (o ascending), masked by the L1-tail CReLU
+    float g2[KQ];
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) g2[i] = 0.0f;
+    if (bvalid) {
+#pragma unroll 2
+        for (int o = 0; o < L2; o += 4) {
+            const float4 d4 = *reinterpret_cast<const float4*>(&s_dl2o[r][o]);
+#pragma unroll
+            for (int i = 0; i < KQ; ++i) {
+                const int k = (int)q + 4 * i;
+                const float4 w4 = *reinterpret_cast<const float4*>(sW2 + (k < LIN ? k : LIN - 1) * WS + o);
+                g2[i] += d4.x * w4.x;
+                g2[i] += d4.y * w4.y;
+                g2[i] += d4.z * w4.z;
+                g2[i] += d4.w * w4.w;
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < KQ; ++i) {
         const int k = (int)q + 4 * i;
         if (k >= LIN) break;
-        float acc = 0.0f;
-        if (bvalid) {
-#pragma unroll
-            for (int o = 0; o < L2; ++o) acc += s_dl2o[r][o] * sW2[o * LIN + k];
-        }
-        s_dl2pre[r][k] = (l2pre[k] > 0.0f && l2pre[k] < 1.0f) ? acc : 0.0f;
+        const float t = s_l1t[r][k < LE ? k : k - LE];
+        const float pre = k < LE ? t * t * a.l1_sqr_scale : t;
+        s_dl2pre[r][k] = (pre > 0.0f && pre < 1.0f) ? g2[i] : 0.0f;
     }
     __syncthreads();
     // L1-tail gradient for this lane's L1 outputs
@@ -449,8 +493,8 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
         float d = 0.0f;
         if (real) {
             if (k < LE) {
-                const float from_sqr = 2.0f * l1t[k] * a.l1_sqr_scale * s_dl2pre[r][k];  // abs_pow2_scale_grad
-                d = s_dl2pre[r][LE + k] + from_sqr;                                        // elementwise_add
+                const float from_sqr = 2.0f * s_l1t[r][k] * a.l1_sqr_scale * s_dl2pre[r][k];  // abs_pow2_scale_grad
+                d = s_dl2pre[r][LE + k] + from_sqr;                                             // elementwise_add
             } else {
                 d = dy;  // slice_scatter_2d of the skip gradient
             }
@@ -460,18 +504,28 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
     }
     __syncthreads();
 
-    // per-tile gradient partials, rows in order (real rows only)
+    // per-tile gradient partials, rows in order (padding rows hold zeros)
     if (bvalid) {
         const TailDims td{(uint32_t)L1, (uint32_t)L2, a.nb};
         const uint32_t cells = td.cells();
         float* part = a.tail_partial + tile * cells;
-        for (uint32_t c = lane; c < cells; c += 64) {
+        // L2 weights: [16 outputs][16 rows] x [16 rows][16 inputs] per MFMA tile
+#pragma unroll
+        for (int ot = 0; ot < L2 / 16; ++ot)
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    acc = mfma4(s_dl2o[4 * c + q][16 * ot + r], s_l2in[4 * c + q][16 * kt + r], acc);
+                const uint32_t k = 16 * kt + r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (k < (uint32_t)LIN) part[(16 * ot + 4 * q + e) * LIN + k] = acc[e];
+            }
+        for (uint32_t c = td.off_b2() + lane; c < cells; c += 64) {
             float acc = 0.0f;
-            if (c < td.off_b2()) {
-                const uint32_t o = c / LIN, k = c % LIN;
-                for (int rr = 0; rr < 16; ++rr)
-                    if (s_real[rr]) acc += s_l2in[rr][k] * s_dl2o[rr][o];
-            } else if (c < td.off_w3()) {
+            if (c < td.off_w3()) {
                 const uint32_t o = c - td.off_b2();
                 for (int rr = 0; rr < 16; ++rr)
                     if (s_real[rr]) acc += s_dl2o[rr][o];
