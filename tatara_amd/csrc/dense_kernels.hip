@@ -310,13 +310,12 @@ __global__ __launch_bounds__(256) void sum_partials_f64_kernel(const double* __r
 // lane reads four outputs' weights at once.  Every
 // per-row sum keeps the reference order (k ascending for L2, o ascending for
 // L3 and for the L2 input gradient); the gradient partials are per tile, rows
-// in order (the L2 weights' as f32 MFMAs over the tile's rows), and are
-// reduced per bucket over the bucket's tiles.
+// in order, and are reduced per bucket over the bucket's tiles.
 //
 // Bound by its chain of LDS round trips.  The L1 outputs as per-lane arrays
 // indexed by lane went to scratch memory at l1 = 32, and every cell of the L2
-// weight gradient read 32 LDS words: l1 32, l2 64, b 2048 88 -> 31 us;
-// l1 16, l2 32, b 65536 70 -> 38 us; l1 8, l2 32, b 16384 22 -> 15 us.
+// weight gradient read 32 LDS words: l1 32, l2 64, b 2048 88 -> 34 us;
+// l1 16, l2 32, b 65536 70 -> 39 us; l1 8, l2 32, b 16384 22 -> 16 us.
 // ---------------------------------------------------------------------------
 template <int L1, int L2>
 __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t train) {
@@ -326,13 +325,12 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
     constexpr int KQ = (LIN + 3) / 4;      // L2 inputs per lane (backward)
     constexpr int JQ = L1 / 4;             // L1 outputs per lane (backward)
     constexpr int WS = L2 + 4;             // row stride of the transposed weights: 16-byte rows, spread banks
-    constexpr int KT = (LIN + 15) / 16;    // 16-input tiles of the L2 weight gradient
-    constexpr int IS = 16 * KT + 1;        // row stride of the L2 inputs (zero past LIN)
-    static_assert(L2 % 16 == 0 && L1 % 4 == 0, "quarters of whole float4, whole MFMA tiles");
+    constexpr int IS = 4 * KQ + 4;         // row stride of the L2 inputs (zero past LIN)
+    static_assert(L2 % 16 == 0 && L1 % 4 == 0, "quarters of whole float4");
     __shared__ __align__(16) float sW2[LIN * WS];  // [k][o]
     __shared__ float sB2[L2], sW3[L2];
     __shared__ float s_l1t[16][L1 + 1];
-    __shared__ float s_l2in[16][IS];
+    __shared__ __align__(16) float s_l2in[16][IS];
     __shared__ float s_l2a[16][L2 + 1];
     __shared__ __align__(16) float s_dl2o[16][WS];
     __shared__ float s_dl2pre[16][LIN + 1];
@@ -396,7 +394,7 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
         }
     }
     if (lane < 16)
-        for (int k = LIN; k < 16 * KT; ++k) s_l2in[lane][k] = 0.0f;
+        for (int k = LIN; k < 4 * KQ; ++k) s_l2in[lane][k] = 0.0f;
     __syncthreads();
     // L2 (dense_mm_fwd_bucket: the sum starts at the bias, k ascending) + CReLU
     float l2o[OQ];
@@ -509,20 +507,27 @@ __global__ __launch_bounds__(64) void ls_tail_kernel(LsDenseArgs a, int32_t trai
         const TailDims td{(uint32_t)L1, (uint32_t)L2, a.nb};
         const uint32_t cells = td.cells();
         float* part = a.tail_partial + tile * cells;
-        // L2 weights: [16 outputs][16 rows] x [16 rows][16 inputs] per MFMA tile
+        // L2 weights: a lane takes cells of 4 outputs x 4 inputs (two 16-byte
+        // LDS reads a row for 16 products)
+        constexpr uint32_t KB = (LIN + 3) / 4;
+        for (uint32_t blk = lane; blk < L2 / 4 * KB; blk += 64) {
+            const uint32_t o = blk / KB * 4, k = blk % KB * 4;
+            floatx4 acc[4];
 #pragma unroll
-        for (int ot = 0; ot < L2 / 16; ++ot)
+            for (int e = 0; e < 4; ++e) acc[e] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+            for (int rr = 0; rr < 16; ++rr) {
+                const floatx4 d = *reinterpret_cast<const floatx4*>(&s_dl2o[rr][o]);
+                const floatx4 x = *reinterpret_cast<const floatx4*>(&s_l2in[rr][k]);
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) {
-                floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    acc = mfma4(s_dl2o[4 * c + q][16 * ot + r], s_l2in[4 * c + q][16 * kt + r], acc);
-                const uint32_t k = 16 * kt + r;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (k < (uint32_t)LIN) part[(16 * ot + 4 * q + e) * LIN + k] = acc[e];
+                for (int e = 0; e < 4; ++e) acc[e] += x * d[e];
             }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (k + j < (uint32_t)LIN) part[(o + e) * LIN + k + j] = acc[e][j];
+        }
         for (uint32_t c = td.off_b2() + lane; c < cells; c += 64) {
             float acc = 0.0f;
             if (c < td.off_w3()) {
@@ -738,7 +743,8 @@ __global__ __launch_bounds__(256) void ls_l1_wgrad_kernel(LsDenseArgs a) {
 // ft_post_perspective_grad_fused), then the pairwise CReLU gradient into dft
 // (native_kernels.cu:2260-2302).  Grid (column block, row block): a wave owns
 // 64 columns of the combined output over post_tiles sorted tiles and writes
-// their ft_b gradient partials per perspective for that row block.  The f16
+// their ft_b gradient partials per perspective: f32 one for every kPostTiles of
+// them, rows in order; f16 one for the row block.  The f16
 // variant reads f16 raw sums and writes the f16 dft, scaled by dft_scale and
 // clamped to +-65504 with a count of every clamp
 // (ft_post_perspective_grad_fused_fp16, native_kernels.cu:2304-2352); the
@@ -753,8 +759,8 @@ __global__ __launch_bounds__(256) void ls_l1_wgrad_kernel(LsDenseArgs a) {
 // 8-byte) pieces.
 // With the sums as per-column FMAs (32 an element, plus the dl1 broadcasts)
 // the kernel was bound by vector issue in f16.  ft_out 1536, b 65536: f16 273
-// -> 193 us (0.8 GB, 4.2 TB/s), f32 324 -> 324 (1.6 GB, 5.0 TB/s: memory);
-// ft_out 512, l1 32, b 2048: 25 -> 15 us.  The weights wait in LDS (each lane
+// -> 193 us (0.8 GB, 4.2 TB/s), f32 324 -> 330 (1.6 GB, 4.9 TB/s: memory);
+// ft_out 512, l1 32, b 2048: 25 -> 18 us.  The weights wait in LDS (each lane
 // reads back what it wrote, so nothing is synchronised): in registers they
 // cost a wave per SIMD.  The next tile's raw sums loaded ahead measured
 // slower (255 us f16): 32 more registers, one wave per SIMD less.
@@ -779,6 +785,8 @@ __global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, ui
     using Raw = typename std::conditional<H16, h4, floatx4>::type;
     // a lane's own weights of the current bucket: [bucket, shared][k][lane]
     __shared__ floatx4 s_w[2][KC][128];
+    // f32: a wave's gradients of a tile, [row][column]
+    __shared__ __align__(16) float s_g[H16 ? 1 : 2][H16 ? 1 : 16][64];
     const uint32_t ft_out = a.ft_out, half = ft_out / 2;
     const uint64_t batch = a.batch;
     const uint32_t tid = threadIdx.x, lane = tid % 64, i = lane % 16, q = lane / 16;
@@ -806,7 +814,12 @@ __global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, ui
         s_w[1][k][tid] = v;
     }
     int32_t cur_bin = -2;
-    floatx4 acc_a = {0.f, 0.f, 0.f, 0.f}, acc_b = {0.f, 0.f, 0.f, 0.f};
+    // ft_b gradients: f32, of the wave's column `lane` and of its partner, rows
+    // in order; f16, of the lane's rows and columns (added up at the end)
+    using Bias = typename std::conditional<H16, floatx4, float>::type;
+    Bias acc_a = {}, acc_b = {};
+    float(*g_t)[64] = s_g[H16 ? 0 : tid / 64];
+    float* pp = a.ftb_partial + persp * ft_out + (H16 ? p : p - 4 * i + lane);
     uint32_t clamps = 0;
     const uint32_t tile0 = blockIdx.y * post_tiles;
     const uint32_t tiles_total = (uint32_t)(a.padded_b / 16);
@@ -862,19 +875,27 @@ __global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, ui
             }
 #pragma unroll
             for (int g = 0; g < 4; ++g) da[g] += db[g];
+            [[maybe_unused]] floatx4 gbs[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                if (rows[r] < 0) continue;
+                if (H16 && rows[r] < 0) continue;
                 floatx4 ga, gb;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float xa = (float)xr[r][g] + ba[g], xb = (float)yr[r][g] + bb[g];
                     const float dy = da[g][r];
-                    ga[g] = (xa > 0.0f && xa < 1.0f) ? dy * crelu01(xb) * a.ft_post_scale : 0.0f;
-                    gb[g] = (xb > 0.0f && xb < 1.0f) ? dy * crelu01(xa) * a.ft_post_scale : 0.0f;
+                    const bool real = H16 || rows[r] >= 0;  // a padding row adds +0.0 (f16: skipped)
+                    ga[g] = (real && xa > 0.0f && xa < 1.0f) ? dy * crelu01(xb) * a.ft_post_scale : 0.0f;
+                    gb[g] = (real && xb > 0.0f && xb < 1.0f) ? dy * crelu01(xa) * a.ft_post_scale : 0.0f;
                 }
-                acc_a += ga;
-                acc_b += gb;
+                if constexpr (H16) {
+                    acc_a += ga;
+                    acc_b += gb;
+                } else {
+                    *reinterpret_cast<floatx4*>(&g_t[4 * q + r][4 * i]) = ga;
+                    gbs[r] = gb;
+                }
+                if (!H16 && rows[r] < 0) continue;
                 const uint64_t row = (uint64_t)rows[r] * kDftChunk;
                 if constexpr (H16) {
                     floatx4 va = ga * a.dft_scale, vb = gb * a.dft_scale;
@@ -897,21 +918,47 @@ __global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, ui
                     dft[(off_b + row) / 4] = gb;
                 }
             }
+            if constexpr (!H16) {
+                // the rows' gradients added in row order, a column per lane,
+                // through the wave's own LDS (a wave's LDS accesses complete
+                // in order)
+                auto in_order = [&](float& acc) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int rr = 0; rr < 16; ++rr) acc += g_t[rr][lane];
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                };
+                in_order(acc_a);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *reinterpret_cast<floatx4*>(&g_t[4 * q + r][4 * i]) = gbs[r];
+                in_order(acc_b);
+            }
+        }
+        if constexpr (!H16) {
+            if ((t + 1) % kPostTiles == 0 || t + 1 == n_tiles) {  // the partial of these kPostTiles tiles
+                float* o = pp + (uint64_t)((tile0 + t) / kPostTiles) * 2 * ft_out;
+                o[0] = acc_a;
+                o[half] = acc_b;
+                acc_a = acc_b = 0.0f;
+            }
         }
         cur = next;
     }
-    // the four lanes of a column run hold different rows' sums
+    if constexpr (H16) {  // the row block's partial: the four lanes of a column run hold different rows' sums
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        acc_a[g] += __shfl_xor(acc_a[g], 16);
-        acc_b[g] += __shfl_xor(acc_b[g], 16);
-        acc_a[g] += __shfl_xor(acc_a[g], 32);
-        acc_b[g] += __shfl_xor(acc_b[g], 32);
-    }
-    if (q == 0) {
-        float* pp = a.ftb_partial + ((uint64_t)blockIdx.y * 2 + persp) * ft_out;
-        *reinterpret_cast<floatx4*>(pp + p) = acc_a;
-        *reinterpret_cast<floatx4*>(pp + p + half) = acc_b;
+        for (int g = 0; g < 4; ++g) {
+            acc_a[g] += __shfl_xor(acc_a[g], 16);
+            acc_b[g] += __shfl_xor(acc_b[g], 16);
+            acc_a[g] += __shfl_xor(acc_a[g], 32);
+            acc_b[g] += __shfl_xor(acc_b[g], 32);
+        }
+        if (q == 0) {
+            float* o = pp + (uint64_t)blockIdx.y * 2 * ft_out;
+            *reinterpret_cast<floatx4*>(o) = acc_a;
+            *reinterpret_cast<floatx4*>(o + half) = acc_b;
+        }
     }
     if (H16 && clamps) atomicAdd(a.clamp_counter, (unsigned long long)clamps);
 }
@@ -1000,11 +1047,14 @@ __global__ __launch_bounds__(256) void ls_dense_finalize_kernel(LsDenseArgs a, G
 }  // namespace
 
 uint32_t ls_tail_workgroups(uint32_t padded_b) { return ceil_div(padded_b, 16); }
-static uint32_t post_tiles(uint32_t padded_b, uint32_t ft_out) { return post_block_tiles(padded_b / 16, ft_out); }
-static uint32_t post_row_blocks(uint32_t padded_b, uint32_t ft_out) {
-    return ceil_div(padded_b / 16, post_tiles(padded_b, ft_out));
+uint32_t ls_post_workgroups(uint32_t padded_b) { return ceil_div(padded_b / 16, kPostTiles); }  // f16: at most
+// Tiles per row block of the input-gradient kernel: eight (a column's weights
+// loaded half as often) where that leaves the chip four waves per SIMD, else
+// four.  Eight against four and sixteen at ft_out 1536 f16, b 65536: 211 /
+// 225 / 216 us; at ft_out 512, l1 32, b 2048: 27 / 17 / 49 us.
+static uint32_t post_block_tiles(uint32_t padded_b, uint32_t ft_out) {
+    return (uint64_t)(padded_b / 16) * (ft_out / 64) >= 8 * 4096 ? 2 * kPostTiles : kPostTiles;
 }
-uint32_t ls_post_workgroups(uint32_t padded_b, uint32_t ft_out) { return post_max_blocks(padded_b / 16, ft_out); }
 uint32_t ls_max_chunks(uint32_t padded_b, uint32_t nb) {
     return ceil_div(padded_b / 16, kChunkTiles) + nb + 1;
 }
@@ -1089,7 +1139,8 @@ int32_t launch_ls_l1_weight_grad(const LsDenseArgs& a, hipStream_t stream) {
 int32_t launch_ls_l1_input_post(const LsDenseArgs& a, hipStream_t stream) {
     TATARA_REQUIRE(!a.dft16 || (a.ft_stm16 && a.ft_nstm16 && a.clamp_counter),
                    "an f16 dft needs the f16 raw sums and a clamp counter");
-    const uint32_t rows = post_row_blocks(a.padded_b, a.ft_out);
+    const uint32_t block_tiles = post_block_tiles(a.padded_b, a.ft_out);
+    const uint32_t rows = ceil_div(a.padded_b / 16, block_tiles);
     if (rows == 0) return kOk;
     TATARA_REQUIRE(a.ft_out % 128 == 0, "ft_out must be a multiple of 128");
     TATARA_REQUIRE(a.l1 == 8 || a.l1 == 16 || a.l1 == 32, kLsDenseShapes);
@@ -1100,7 +1151,7 @@ int32_t launch_ls_l1_input_post(const LsDenseArgs& a, hipStream_t stream) {
                           : (a.l1 == 32   ? ls_l1_input_post_kernel<32, false>
                              : a.l1 == 16 ? ls_l1_input_post_kernel<16, false>
                                           : ls_l1_input_post_kernel<8, false>);
-    kernel<<<grid, 128, 0, stream>>>(a, post_tiles(a.padded_b, a.ft_out));
+    kernel<<<grid, 128, 0, stream>>>(a, block_tiles);
     TATARA_LAUNCHED("ls_l1_input_post");
     return kOk;
 }
@@ -1117,7 +1168,8 @@ int32_t launch_ls_dense_finalize(const LsDenseArgs& a, LsDenseGroup* groups,
     const uint64_t n = gt.start[9];
     const TailDims td{a.l1, a.l2, a.nb};
     const uint32_t n_tail = ls_tail_workgroups(a.padded_b);
-    const uint32_t n_post = post_row_blocks(a.padded_b, a.ft_out);
+    const uint32_t n_post =
+        a.dft16 ? ceil_div(a.padded_b / 16, post_block_tiles(a.padded_b, a.ft_out)) : ls_post_workgroups(a.padded_b);
     // bucket g's tile partials are the rows [tail_seg[g], tail_seg[g + 1])
     reduce_rows(a.tail_partial, n_tail, td.cells(), a.tail_seg, a.nb, a.tail_sum, stream);
     reduce_rows(a.b1s_partial, n_tail, a.l1, nullptr, 1, a.b1s_sum, stream);

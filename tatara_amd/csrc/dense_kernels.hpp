@@ -31,25 +31,7 @@ struct TailDims {
 };
 
 constexpr uint32_t kChunkTiles = 16;     // 16-row tiles per L1 weight-gradient chunk
-// Row blocks of the L1-input/FT-post kernels (a wave: 64 columns of a block's
-// 16-row tiles).  Tiles per row block: as many as leave the chip four waves per SIMD,
-// at most eight.  Longer blocks load each column's weights less often; shorter
-// ones fill the chip.  One tile against four and eight at LayerStack ft_out 512,
-// l1 32, b 2048: 15.4 / 16.6 / 27.2 us; eight against four and sixteen at
-// ft_out 1536 f16, b 65536: 211 / 225 / 216 us.
-constexpr uint32_t kPostWaves = 4096;
-inline uint32_t post_block_tiles(uint32_t tiles, uint32_t ft_out) {
-    const uint64_t waves = (uint64_t)tiles * ((ft_out + 63) / 64);
-    return (uint32_t)(waves >= 8 * kPostWaves ? 8 : waves >= kPostWaves ? waves / kPostWaves : 1);
-}
-// The most row blocks of any batch of up to `tiles` tiles: its own, or those of
-// the largest batch that still takes one tile per block.
-inline uint32_t post_max_blocks(uint32_t tiles, uint32_t ft_out) {
-    const uint32_t t = post_block_tiles(tiles, ft_out), own = (tiles + t - 1) / t;
-    const uint32_t peak = 2 * kPostWaves / ((ft_out + 63) / 64) + 1;
-    const uint32_t most = peak < tiles ? peak : tiles;
-    return own > most ? own : most;
-}
+constexpr uint32_t kPostTiles = 4;       // 16-row tiles per ft_b partial of the L1-input/FT-post kernel
 
 struct LsDenseArgs {
     // shapes
@@ -124,8 +106,7 @@ struct LsDenseArgs {
 };
 
 uint32_t ls_tail_workgroups(uint32_t padded_b);
-// row blocks (ft_b partials) of the input-gradient kernel, at most, up to padded_b
-uint32_t ls_post_workgroups(uint32_t padded_b, uint32_t ft_out);
+uint32_t ls_post_workgroups(uint32_t padded_b);  // ft_b partials
 uint32_t ls_max_chunks(uint32_t padded_b, uint32_t nb);
 
 // Forward: L1 (bucket + shared) on sorted tiles.

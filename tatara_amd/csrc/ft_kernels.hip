@@ -1957,14 +1957,16 @@ bool ft_forward_block_ok(int mode, bool f16_table, uint32_t ft_out, uint32_t pie
 //      71.5       856 / 967  473 / 615  358 / 356  319 / 311
 //     143                    705 / 1002 539 / 572  550 / 513
 //   occurrences   Simple 256 Simple 512 Simple 1024 (f32, concat)
-//       2.6       202 / 134  374 / 257  759 / 534
-//      20.9       277 / 244  480 / 464  926 / 959
-//      41.8       346 / 351  596 / 671  1176 / 1341
+//       2.5       202 / 134  374 / 257  759 / 534
+//      19.9       277 / 244  480 / 464  926 / 959
+//      39.7       346 / 351  596 / 671  1176 / 1341
+// (and at 39.7, Simple 256, the L1 forward after the staged form finds more of
+// `combined` in the cache: 102 against 131).
 bool ft_forward_block_pays(int mode, bool f16_table, uint32_t ft_out, uint32_t cols, uint32_t max_active,
                            uint32_t batch) {
     uint64_t line;  // occurrences per table row
     if (mode == kConcat) {
-        line = ft_out <= 256 ? 40 : 20;
+        line = ft_out <= 256 ? 32 : 20;
     } else {
         if (ft_out <= 256) return false;
         line = f16_table ? (ft_out <= 512 ? 80 : 20) : (ft_out < 768 ? 20 : 16);

@@ -297,92 +297,88 @@ __global__ __launch_bounds__(256) void simple_l1_wgrad_kernel(SimpleDenseArgs a)
 // dcombined[row][p*ft_out + c] = sum_o dl1[row][o] * l1_w[p*ft_out + c][o] (o
 // ascending, from 0), then dft_p[row][c] passes it where 0 < x < 1
 // (simple_bwd_ft_act_crelu_fused, native_kernels.cu:1452).  The ft_b partial
-// adds stm + nstm per row (simple_bias_grad_dual, native_kernels.cu:1572).
+// adds stm + nstm per row, the block's rows in order (simple_bias_grad_dual,
+// native_kernels.cu:1572).
 //
-// A wave owns 64 FT columns of both perspectives over a row block's 16-row
-// tiles, the products on the matrix cores in the layout of
-// ls_l1_input_post_kernel: column group g's column l%16 is the wave's column
-// 4 * (l%16) + g, so a lane ends with four rows of four consecutive columns and
-// moves x and dft in 16-byte pieces.  One thread per column with its 2 * L1
-// weights in registers was bound by vector issue, and by too few waves for
-// small batches (256x2-32-32, b 4096: 50 -> 14 us).
+// A workgroup: 64 FT columns of both perspectives x kSimplePostRows rows, wave
+// w a quarter of the rows, a lane one column with its weights in registers.
+// The waves add their rows' sums to the ft_b partial in turn.  Bound by its
+// multiplies and adds (2 * l1 unfused products an element and perspective) and,
+// for small batches, by waves in flight: with a workgroup of 256 columns and
+// every row in one wave 256x2-32-32 at b 4096 had 256 waves and took 50 us,
+// now 13 us.
 // ---------------------------------------------------------------------------
 template <int L1>
-__global__ __launch_bounds__(64) void simple_l1_input_post_kernel(SimpleDenseArgs a, uint32_t block_tiles) {
-    constexpr int KC = L1 / 4;  // MFMAs per column group and perspective
-    __shared__ floatx4 s_w[2][KC][64];  // a lane's own weights: [perspective][k][lane]
+__global__ __launch_bounds__(256) void simple_l1_input_post_kernel(SimpleDenseArgs a) {
+    constexpr int R = kSimplePostRows, RW = R / 4;
+    __shared__ __align__(16) float s_d[R][L1];
+    __shared__ float s_acc[64];
     const uint32_t ft_out = a.ft_out, batch = a.batch;
-    const uint32_t lane = threadIdx.x, i = lane % 16, q = lane / 16;
-    const uint32_t c = blockIdx.x * 64 + 4 * i;
-    // ft_out % 32 == 0: a lane's run of four lies wholly within the row or past it
+    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const uint32_t r0 = blockIdx.y * R;
+    const uint32_t nr = min((uint32_t)R, batch - r0);
+    for (uint32_t e = threadIdx.x; e < (uint32_t)(R * L1); e += 256)
+        s_d[e / L1][e % L1] = e / L1 < nr ? a.dl1[(uint64_t)r0 * L1 + e] : 0.0f;
+    const uint32_t c = blockIdx.x * 64 + lane;
     const bool cvalid = c < ft_out;
     const uint32_t cc = cvalid ? c : 0;
+    float ws[L1], wn[L1];
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int k = 0; k < KC; ++k) {
-            floatx4 v;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) v[g] = a.l1_w[(uint64_t)(p * ft_out + cc + g) * L1 + 4 * k + q];
-            s_w[p][k][lane] = v;
-        }
+    for (int o = 0; o < L1; o += 4) {
+        const float4 s = *reinterpret_cast<const float4*>(a.l1_w + (uint64_t)cc * L1 + o);
+        const float4 n = *reinterpret_cast<const float4*>(a.l1_w + (uint64_t)(ft_out + cc) * L1 + o);
+        ws[o] = s.x, ws[o + 1] = s.y, ws[o + 2] = s.z, ws[o + 3] = s.w;
+        wn[o] = n.x, wn[o + 1] = n.y, wn[o + 2] = n.z, wn[o + 3] = n.w;
+    }
+    __syncthreads();
     // chunk-major dft: column c of row r at (c / 256) * 2*batch*256 + r * 256 + c % 256
     const uint64_t cbase = (uint64_t)(cc / kDftChunk) * 2 * batch * kDftChunk + cc % kDftChunk;
     float* dft_s = a.dft + cbase;
     float* dft_n = a.dft + cbase + (uint64_t)batch * kDftChunk;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    const uint32_t tile0 = blockIdx.y * block_tiles, tiles = (batch + 15) / 16;
-    const uint32_t tile1 = tile0 + block_tiles < tiles ? tile0 + block_tiles : tiles;
-    for (uint32_t tile = tile0; tile < tile1; ++tile) {
-        const uint32_t row_d = tile * 16 + i;
-        float d[KC];  // dl1 of row i of the tile (0 past the batch), o = 4k + q
+    const uint32_t w0 = wave * RW;  // the wave's first row of the block
+    float xs[RW], xn[RW], both[RW];
 #pragma unroll
-        for (int k = 0; k < KC; ++k) {
-            const float v = a.dl1[(uint64_t)(row_d < batch ? row_d : 0) * L1 + 4 * k + q];
-            d[k] = row_d < batch ? v : 0.0f;
+    for (int r = 0; r < RW; ++r) {  // row 0 (always valid) past the batch
+        const uint64_t i = (uint64_t)(w0 + r < nr ? r0 + w0 + r : 0) * ft_out + cc;
+        xs[r] = a.ft_stm[i];
+        xn[r] = a.ft_nstm[i];
+    }
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        float da = 0.0f, db = 0.0f;
+#pragma unroll
+        for (int o = 0; o < L1; o += 4) {
+            const float4 d = *reinterpret_cast<const float4*>(&s_d[w0 + r][o]);
+            da += d.x * ws[o];
+            db += d.x * wn[o];
+            da += d.y * ws[o + 1];
+            db += d.y * wn[o + 1];
+            da += d.z * ws[o + 2];
+            db += d.z * wn[o + 2];
+            da += d.w * ws[o + 3];
+            db += d.w * wn[o + 3];
         }
-        const uint32_t row0 = tile * 16 + 4 * q;
-        floatx4 xs[4], xn[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {  // row 0 (always valid) past the batch
-            const uint64_t at = (uint64_t)(row0 + r < batch ? row0 + r : 0) * ft_out + cc;
-            xs[r] = *reinterpret_cast<const floatx4*>(a.ft_stm + at);
-            xn[r] = *reinterpret_cast<const floatx4*>(a.ft_nstm + at);
-        }
-        floatx4 ds[4], dn[4];  // [column group][row]
-#pragma unroll
-        for (int g = 0; g < 4; ++g) ds[g] = dn[g] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KC; ++k) {
-            const floatx4 w_s = s_w[0][k][lane], w_n = s_w[1][k][lane];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                ds[g] = mfma4(d[k], w_s[g], ds[g]);
-                dn[g] = mfma4(d[k], w_n[g], dn[g]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (row0 + r >= batch || !cvalid) continue;
-            floatx4 gs, gn;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                gs[g] = (xs[r][g] > 0.0f && xs[r][g] < 1.0f) ? ds[g][r] : 0.0f;
-                gn[g] = (xn[r][g] > 0.0f && xn[r][g] < 1.0f) ? dn[g][r] : 0.0f;
-            }
-            const uint64_t di = (uint64_t)(row0 + r) * kDftChunk;
-            *reinterpret_cast<floatx4*>(dft_s + di) = gs;
-            *reinterpret_cast<floatx4*>(dft_n + di) = gn;
-            acc += gs + gn;
+        const float gs = (xs[r] > 0.0f && xs[r] < 1.0f) ? da : 0.0f;
+        const float gn = (xn[r] > 0.0f && xn[r] < 1.0f) ? db : 0.0f;
+        both[r] = gs + gn;
+        if (cvalid && w0 + r < nr) {
+            const uint64_t di = (uint64_t)(r0 + w0 + r) * kDftChunk;
+            dft_s[di] = gs;
+            dft_n[di] = gn;
         }
     }
-    // the four lanes of a column run hold different rows' sums
+    // the block's rows in order: wave after wave
+    for (uint32_t w = 0; w < 4; ++w) {
+        if (wave == w) {
+            float acc = w ? s_acc[lane] : 0.0f;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        acc[g] += __shfl_xor(acc[g], 16);
-        acc[g] += __shfl_xor(acc[g], 32);
+            for (int r = 0; r < RW; ++r)
+                if (w0 + r < nr) acc += both[r];
+            s_acc[lane] = acc;
+        }
+        __syncthreads();
     }
-    if (q == 0 && cvalid) *reinterpret_cast<floatx4*>(a.ftb_partial + (uint64_t)blockIdx.y * ft_out + c) = acc;
+    if (wave == 0 && cvalid) a.ftb_partial[(uint64_t)blockIdx.y * ft_out + c] = s_acc[lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -436,11 +432,7 @@ __global__ __launch_bounds__(256) void simple_dense_finalize_kernel(SimpleDenseA
 
 uint32_t simple_tail_workgroups(uint32_t batch) { return ceil_div(batch, 16); }
 uint32_t simple_chunks(uint32_t batch) { return ceil_div(batch, kSimpleChunkRows); }
-uint32_t simple_post_workgroups(uint32_t batch, uint32_t ft_out) { return post_max_blocks(ceil_div(batch, 16), ft_out); }
-static uint32_t post_row_blocks(uint32_t batch, uint32_t ft_out) {
-    const uint32_t tiles = ceil_div(batch, 16);
-    return ceil_div(tiles, post_block_tiles(tiles, ft_out));
-}
+uint32_t simple_post_workgroups(uint32_t batch) { return ceil_div(batch, kSimplePostRows); }
 
 static int32_t check_dims(const SimpleDenseArgs& a) {
     TATARA_REQUIRE(simple_dense_shape_ok(a.l1, a.l2), kSimpleDenseShapes);
@@ -509,9 +501,10 @@ int32_t launch_simple_l1_weight_grad(const SimpleDenseArgs& a, hipStream_t strea
 int32_t launch_simple_l1_input_post(const SimpleDenseArgs& a, hipStream_t stream) {
     int32_t st = check_dims(a);
     if (st) return st;
-    if (a.batch == 0) return kOk;
-    const dim3 grid(ceil_div(a.ft_out, 64), post_row_blocks(a.batch, a.ft_out));
-    TATARA_BY_L1(simple_l1_input_post_kernel, grid, 64, a, post_block_tiles(ceil_div(a.batch, 16), a.ft_out));
+    const uint32_t rows = simple_post_workgroups(a.batch);
+    if (rows == 0) return kOk;
+    const dim3 grid(ceil_div(a.ft_out, 64), rows);
+    TATARA_BY_L1(simple_l1_input_post_kernel, grid, 256, a);
     TATARA_LAUNCHED("simple_l1_input_post");
     return kOk;
 }
@@ -529,7 +522,7 @@ int32_t launch_simple_dense_finalize(const SimpleDenseArgs& a, SimpleDenseGroup*
     if ((st = launch_reduce_rows(a.w1_partial, simple_chunks(a.batch), K * a.l1, nullptr, 1, a.w1_sum,
                                  stream)))
         return st;
-    if ((st = launch_reduce_rows(a.ftb_partial, post_row_blocks(a.batch, a.ft_out), a.ft_out, nullptr, 1,
+    if ((st = launch_reduce_rows(a.ftb_partial, simple_post_workgroups(a.batch), a.ft_out, nullptr, 1,
                                  a.ftb_sum, stream)))
         return st;
     SimpleGroupTable gt;

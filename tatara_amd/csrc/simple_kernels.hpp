@@ -30,6 +30,7 @@ struct SimpleTailDims {
 };
 
 constexpr uint32_t kSimpleChunkRows = 256;   // rows per L1 weight-gradient chunk
+constexpr uint32_t kSimplePostRows = 64;     // rows per L1-input/FT-post workgroup (an ft_b partial)
 
 struct SimpleDenseArgs {
     uint32_t batch, ft_out, l1, l2;
@@ -63,8 +64,7 @@ struct SimpleDenseArgs {
 
 uint32_t simple_tail_workgroups(uint32_t batch);
 uint32_t simple_chunks(uint32_t batch);
-// row blocks (ft_b partials) of the input-gradient kernel, at most, up to batch
-uint32_t simple_post_workgroups(uint32_t batch, uint32_t ft_out);
+uint32_t simple_post_workgroups(uint32_t batch);
 
 // L1 forward (MFMA): l1_pre = combined . l1_w + l1_b.
 int32_t launch_simple_l1_forward(const SimpleDenseArgs& a, hipStream_t stream);

@@ -185,7 +185,7 @@ class SimpleTrainer final : public TrainerBase {
             return st;
         const SimpleTailDims td{l1, l2};
         const uint64_t n_tail = simple_tail_workgroups(max_b), n_chunks = simple_chunks(max_b),
-                       n_post = simple_post_workgroups(max_b, ft_out);
+                       n_post = simple_post_workgroups(max_b);
         if ((st = arena.alloc(&tail_partial, n_tail * td.cells())) ||
             (st = arena.alloc(&w1_partial, n_chunks * K * l1)) ||
             (st = arena.alloc(&ftb_partial, n_post * ft_out)) || (st = arena.alloc(&tail_sum, td.cells())) ||

@@ -267,7 +267,7 @@ class LayerStackTrainer final : public TrainerBase {
             (st = arena.alloc(&dl1_sorted, P * l1)) || (st = arena.alloc(&net_out, B)))
             return st;
         const TailDims td{l1, l2, nb};
-        const uint64_t n_tail = ls_tail_workgroups(max_p), n_post = ls_post_workgroups(max_p, ft_out);
+        const uint64_t n_tail = ls_tail_workgroups(max_p), n_post = ls_post_workgroups(max_p);
         max_chunks = ls_max_chunks(max_p, nb);
         if ((st = arena.alloc(&tail_partial, n_tail * td.cells())) || (st = arena.alloc(&tail_seg, nb + 1)) ||
             (st = arena.alloc(&b1s_partial, n_tail * l1)) || (st = arena.alloc(&loss_partial, n_tail)) ||

@@ -53,7 +53,7 @@ def test_layerstack_forward_on_both_sides(gpu, mixed, kb, pi, ma, ft_out, line):
             assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
 
 
-@pytest.mark.parametrize("kb,pi,ma,ft_out,line", [(10, 64, 44, 256, 40), (10, 64, 38, 512, 20), (2, 1791, 40, 128, 40)])
+@pytest.mark.parametrize("kb,pi,ma,ft_out,line", [(10, 64, 44, 256, 32), (10, 64, 38, 512, 20), (2, 1791, 40, 128, 32)])
 def test_simple_forward_on_both_sides(gpu, kb, pi, ma, ft_out, line):
     spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
     sh = osi.SimpleShape(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, l1=32, l2=32)
