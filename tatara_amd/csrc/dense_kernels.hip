@@ -184,6 +184,80 @@ __global__ __launch_bounds__(256) void ls_l1_fwd_kernel(LsDenseArgs a) {
     }
 }
 
+// The f32 L1 forward for batches of few tiles: a workgroup takes one tile, each
+// of its 2 * NJ waves one of the tile's sums (bucket or shared, 16 outputs) over
+// the whole K in the same order, so the sums are the two-tile kernel's bit for
+// bit (split over K they would not be).  With one wave per two tiles such a
+// batch leaves most SIMDs without a wave, and a wave waits for the loads of two
+// to four K blocks at a time; here eight K blocks are loaded while the eight before
+// them are multiplied.
+template <int NJ>
+__global__ __launch_bounds__(2 * NJ * 64) void ls_l1_fwd_sums_kernel(LsDenseArgs a) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const uint32_t i = lane % 16, q = lane / 16;
+    const uint32_t ft_out = a.ft_out, l1 = a.l1, tile = blockIdx.x;
+    const int32_t bin = scalar_load(a.sorted_bin + (uint64_t)tile * 16);
+    if (bin < 0) return;  // a trailing all-padding tile
+    const bool shared = wave & 1u;
+    const bool bvalid = (uint32_t)bin < a.nb;
+    // unconditional loads from always-valid addresses, masked afterwards
+    const int32_t orig = a.perm[tile * 16 + i];
+    const bool xvalid = orig >= 0;
+    const float4* X = reinterpret_cast<const float4*>(a.combined + (uint64_t)(xvalid ? orig : 0) * ft_out);
+    const uint32_t j = 16 * (wave / 2) + i;
+    const bool jvalid = j < l1, wvalid = jvalid && (shared || bvalid);
+    const uint32_t ic = jvalid ? j : l1 - 1;
+    const float4* W1 = reinterpret_cast<const float4*>(a.l1_w + ((uint64_t)(bvalid ? bin : 0) * l1 + ic) * ft_out);
+    const float* Ws = a.l1s_w + ic;
+    const float b0 = !shared && wvalid ? a.l1_b[bin * l1 + j] : 0.0f;
+    floatx4 acc = {b0, b0, b0, b0};
+    const uint32_t nk = ft_out / 16;
+    constexpr uint32_t kU = 8;
+    struct Group {
+        float4 x[kU], w[kU];
+    };
+    auto load = [&](uint32_t kb0, Group& g) {  // past the end: the last block again, unused
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            const uint32_t kb = kb0 + u < nk ? kb0 + u : nk - 1;
+            g.x[u] = X[kb * 4 + q];
+            if (shared) {
+                const float* w = Ws + (uint64_t)(kb * 16 + 4 * q) * l1;
+                g.w[u] = make_float4(w[0], w[l1], w[2 * l1], w[3 * l1]);
+            } else {
+                g.w[u] = W1[kb * 4 + q];
+            }
+        }
+    };
+    auto multiply = [&](uint32_t kb0, const Group& g) {
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            if (kb0 + u >= nk) break;
+            const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 x = xvalid ? g.x[u] : zero4, w = wvalid ? g.w[u] : zero4;
+            acc = mfma4(x.x, w.x, acc);
+            acc = mfma4(x.y, w.y, acc);
+            acc = mfma4(x.z, w.z, acc);
+            acc = mfma4(x.w, w.w, acc);
+        }
+    };
+    Group g0, g1;
+    load(0, g0);
+    for (uint32_t kb0 = 0; kb0 < nk; kb0 += 2 * kU) {
+        load(kb0 + kU, g1);
+        multiply(kb0, g0);
+        load(kb0 + 2 * kU, g0);
+        multiply(kb0 + kU, g1);
+    }
+    if (!jvalid) return;
+    const float bs = shared ? a.l1s_b[j] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint64_t row = (uint64_t)tile * 16 + 4 * q + r;
+        a.l1_sorted[row * 2 * l1 + (shared ? l1 : 0) + j] = shared ? acc[r] + bs : (bvalid ? acc[r] : 0.0f);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // L1 forward with TF32-class products: f16 operands on the matrix cores
 // (v_mfma_f32_16x16x32_f16, f32 sums).  Lane l supplies A[l%16][8(l/16)+e]
@@ -1059,6 +1133,16 @@ uint32_t ls_max_chunks(uint32_t padded_b, uint32_t nb) {
     return ceil_div(padded_b / 16, kChunkTiles) + nb + 1;
 }
 
+// Tiles from which the f32 L1 forward gives a wave two whole tiles (weights
+// loaded once for 32 rows) instead of a workgroup one tile.  Dense forward
+// phase, two tiles a wave / a workgroup a tile, in us:
+//   b        ft 1536 l1 16   ft 768 l1 8   ft 512 l1 32   ft 256 l1 16
+//   1024       96 / 45         59 / 31       77 / 47        39 / 30
+//   4096      102 / 72         63 / 46       80 / 65        43 / 39
+//   8192      123 / 99         75 / 60       90 / 79        48 / 45
+//   16384     131 / 147        80 / 81       99 / 114       50 / 58
+constexpr uint32_t kL1PairTiles = 640;
+
 int32_t launch_ls_l1_forward(const LsDenseArgs& a, hipStream_t stream) {
     TATARA_REQUIRE(a.l1 >= 2 && a.l1 <= 32, "l1 must be in [2, 32]");
     TATARA_REQUIRE(a.ft_out % 64 == 0, "ft_out must be a multiple of 64");
@@ -1074,6 +1158,11 @@ int32_t launch_ls_l1_forward(const LsDenseArgs& a, hipStream_t stream) {
             ls_l1_fwd_tf32_kernel<2><<<ceil_div(tiles, 4), 256, 0, stream>>>(a);
         else
             ls_l1_fwd_tf32_kernel<1><<<ceil_div(tiles, 4), 256, 0, stream>>>(a);
+    } else if (tiles < kL1PairTiles) {
+        if (two)
+            ls_l1_fwd_sums_kernel<2><<<tiles, 256, 0, stream>>>(a);
+        else
+            ls_l1_fwd_sums_kernel<1><<<tiles, 128, 0, stream>>>(a);
     } else if (two) {
         ls_l1_fwd_kernel<2><<<ceil_div(tiles, 8), 256, 0, stream>>>(a);
     } else {
