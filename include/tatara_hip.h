@@ -269,8 +269,7 @@ TATARA_API int32_t tatara_feature_set_info(int32_t feature_set, int32_t* king_bu
  * kingrank9.rs:11-23, or KP-absolute progress with num_buckets in [1, 256] and
  * the 81*1548 progress weights as f32, progress_kpabs.rs:106-170; f64 file
  * values are rounded to nearest f32 as load_from_bin does).  All pointers are
- * device memory; bucket_idx may be NULL.  Decoded on the GPU, one thread per
- * record; synchronous. */
+ * device memory; bucket_idx may be NULL.  Decoded on the GPU; synchronous. */
 TATARA_API int32_t tatara_psv_to_batch(const uint8_t* psv, int32_t n, int32_t feature_set,
                                        int32_t bucket_mode, int32_t num_buckets,
                                        const float* progress_weights, int32_t* stm_indices,

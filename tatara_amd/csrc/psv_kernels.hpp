@@ -7,8 +7,6 @@
 
 namespace tatara {
 
-constexpr int kPsvThreads = 64;  // records per workgroup
-
 // FeatureSetSpec of the five public feature sets
 // (crates/shogi-features/src/feature_set.rs:103-185).
 struct FeatureSetShape {
