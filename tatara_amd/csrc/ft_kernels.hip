@@ -1289,7 +1289,11 @@ __global__ __launch_bounds__(256) void ft_scan_tables_kernel(FtBlockScan s, Scan
 // round-robin, so wave w owns the group's features w, w + 8, w + 16, ...
 // and adjacent (often equally frequent) features land on different waves,
 // which evens out the hits per wave and stage that the barrier waits for.
-template <bool HDFT, bool HSTATE, bool DEALT>
+//
+// STRIDED: dft rows at a.dft_row_stride (row-major, whole chunks), for a caller
+// whose dft is its own; else the chunk-major rows of kDftChunk values, whose
+// addresses are a shift.
+template <bool HDFT, bool HSTATE, bool DEALT, bool STRIDED = false>
 __global__ __launch_bounds__(kScanWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void ft_grad_scan_kernel(
     FtGradArgs a, FtBlockScan s, ScanGeom geom) {
     constexpr int R = kScanStage, RPW = kScanStage / kScanWaves;
@@ -1345,7 +1349,8 @@ __global__ __launch_bounds__(kScanWaves * 64) __attribute__((amdgpu_waves_per_eu
         return smask[(uint64_t)(T < last ? T : last) * geom.words * kScanFeat];
     };
     auto dft_row = [&](uint32_t row_lanes, uint32_t j) -> const Row4* {
-        return dft4 + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(row_lanes, j % R) * (kDftChunk / 4);
+        const uint64_t row = (uint32_t)__builtin_amdgcn_readlane(row_lanes, j % R);
+        return dft4 + row * (STRIDED ? a.dft_row_stride / 4 : kDftChunk / 4);
     };
 
     float4 acc[kScanFeat];
@@ -1536,7 +1541,7 @@ __device__ __forceinline__ half8 hit_operand(uint32_t b) {
     return __builtin_bit_cast(half8, r);
 }
 
-template <bool HSTATE>
+template <bool HSTATE, bool STRIDED = false>
 __global__ __launch_bounds__(kMfmaWaves * 64) void ft_grad_mfma_kernel(FtGradArgs a, FtBlockScan s,
                                                                        ScanGeom geom) {
     constexpr uint32_t R = kMfmaRows, KS = R / 32, RW = R / kMfmaWaves;  // MFMA steps, rows per wave
@@ -1569,6 +1574,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void ft_grad_mfma_kernel(FtGradArg
     const uint32_t n = na + (s.sched_start[s.n_blocks + K + 1] - b0);
     const _Float16* d16 =
         reinterpret_cast<const _Float16*>(a.dft16) + (uint64_t)chunk * a.dft_chunk_stride + half * kMfmaCols;
+    const uint64_t row_stride = STRIDED ? a.dft_row_stride : kDftChunk;
     // Thread t loads slot mask t of a stage: K-step t / 128, mask word
     // (t / 16) % 8 of the group, feature t % 16, from the stage tables (the
     // block's 32-row stages; a K-step past them has no hits).
@@ -1605,7 +1611,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void ft_grad_mfma_kernel(FtGradArg
         for (uint32_t j = 0; j < RW; ++j) {
             const uint32_t jj = T * R + wave * RW + j;
             const uint64_t r = (uint32_t)__builtin_amdgcn_readlane(pos, wave * RW + j);
-            S.r[j] = jj < n ? reinterpret_cast<const uint32_t*>(d16 + r * kDftChunk)[lane] : 0u;
+            S.r[j] = jj < n ? reinterpret_cast<const uint32_t*>(d16 + r * row_stride)[lane] : 0u;
         }
         const uint32_t ts = T * KS + mks;
         S.mt = ts < n32 ? tmask[(uint64_t)(sb + ts) * geom.words * kScanFeat] : 0u;
@@ -1697,7 +1703,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void ft_grad_mfma_kernel(FtGradArg
             while (mk) {  // the lane's hits, in row order
                 const uint32_t e = __builtin_ctz(mk);
                 mk &= mk - 1;
-                const _Float16* dr = d16 + (uint64_t)tr[e] * kDftChunk + m;
+                const _Float16* dr = d16 + (uint64_t)tr[e] * row_stride + m;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) sum[j] += (float)dr[16 * j];
             }
@@ -2243,12 +2249,23 @@ int32_t launch_ft_scan_tables(const FtBlockScan& s, hipStream_t stream) {
     return kOk;
 }
 
+// The dft layouts of the block scan and its matrix-core form: the trainers'
+// chunk-major one, or (gradients only) a caller's row-major one in whole chunks,
+// which spares it a copy: 100 MB of dft took 60 us at 4 bytes a lane.
+static bool dft_chunk_major(const FtGradArgs& a, uint32_t batch) {
+    return a.dft_row_stride == kDftChunk && a.dft_chunk_stride == 2ull * batch * kDftChunk;
+}
+static bool dft_strided(const FtGradArgs& a) {
+    return a.dft_row_stride == a.ft_out && a.dft_chunk_stride == kDftChunk && a.ft_out % kDftChunk == 0 &&
+           !a.apply_update && !a.m16;
+}
+
 int32_t launch_ft_grad_scan(const FtGradArgs& a, const FtBlockScan& s, hipStream_t stream, bool fallback) {
     TATARA_REQUIRE(ft_scan_mask_words(s.piece_inputs) > 0, "block scan: piece_inputs out of range");
     TATARA_REQUIRE(s.stage_rows && s.stage_masks, "block scan: stage tables (launch_ft_scan_tables)");
     TATARA_REQUIRE((a.dft != nullptr) != (a.dft16 != nullptr), "block scan: one dft (f32 or f16)");
-    TATARA_REQUIRE(a.dft_row_stride == kDftChunk && a.dft_chunk_stride == 2ull * s.batch * kDftChunk,
-                   "block scan: chunk-major dft");
+    const bool strided = dft_strided(a);
+    TATARA_REQUIRE(strided || dft_chunk_major(a, s.batch), "block scan: chunk-major dft, or row-major in whole chunks");
     TATARA_REQUIRE(a.ft_out % 4 == 0 && a.rows == s.cols, "block scan: shapes");
     TATARA_REQUIRE(moment_scales_ok(a), "f16 moment scales must be powers of two");
     const ScanGeom geom = scan_geom(s.piece_inputs);
@@ -2268,7 +2285,13 @@ int32_t launch_ft_grad_scan(const FtGradArgs& a, const FtBlockScan& s, hipStream
         else                                                                            \
             ft_grad_scan_kernel<false, false, D><<<g, t, 0, stream>>>(a, s, geom);      \
     } while (0)
-        if (s.dealt)
+        if (strided) {
+            TATARA_REQUIRE(s.dealt, "block scan: row-major dft takes dealt stage tables");
+            if (a.dft16)
+                ft_grad_scan_kernel<true, false, true, true><<<g, t, 0, stream>>>(a, s, geom);
+            else
+                ft_grad_scan_kernel<false, false, true, true><<<g, t, 0, stream>>>(a, s, geom);
+        } else if (s.dealt)
             TATARA_SCAN(true);
         else
             TATARA_SCAN(false);
@@ -2285,8 +2308,8 @@ int32_t launch_ft_grad_mfma(const FtGradArgs& a, const FtBlockScan& s, hipStream
     TATARA_REQUIRE(s.stage_rows && s.stage_masks, "block scan: stage tables (launch_ft_scan_tables)");
     TATARA_REQUIRE(ft_scan_mask_words(s.piece_inputs) > 0, "mfma backward: piece_inputs out of range");
     TATARA_REQUIRE(a.dft16 && !a.dft, "mfma backward: f16 dft only");
-    TATARA_REQUIRE(a.dft_row_stride == kDftChunk && a.dft_chunk_stride == 2ull * s.batch * kDftChunk,
-                   "mfma backward: chunk-major dft");
+    const bool strided = dft_strided(a);
+    TATARA_REQUIRE(strided || dft_chunk_major(a, s.batch), "mfma backward: chunk-major dft, or row-major in whole chunks");
     TATARA_REQUIRE(a.ft_out % 4 == 0 && a.rows == s.cols, "mfma backward: shapes");
     TATARA_REQUIRE(moment_scales_ok(a), "f16 moment scales must be powers of two");
     TATARA_REQUIRE(s.n_blocks <= 128, "mfma backward: at most 128 king blocks");
@@ -2297,7 +2320,9 @@ int32_t launch_ft_grad_mfma(const FtGradArgs& a, const FtBlockScan& s, hipStream
     const uint64_t grid = (pairs + kNumXcd - 1) / kNumXcd * kNumXcd * geom.n_groups * 2;
     if (grid > 0) {
         const uint32_t t = kMfmaWaves * 64;
-        if (a.m16)
+        if (strided)
+            ft_grad_mfma_kernel<false, true><<<(uint32_t)grid, t, 0, stream>>>(a, s, geom);
+        else if (a.m16)
             ft_grad_mfma_kernel<true><<<(uint32_t)grid, t, 0, stream>>>(a, s, geom);
         else
             ft_grad_mfma_kernel<false><<<(uint32_t)grid, t, 0, stream>>>(a, s, geom);

@@ -9,6 +9,7 @@
 
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/tatara_hip.h"
@@ -56,15 +57,64 @@ struct DevScratch {
     }
 };
 
-// row-major [rows][ft_out] -> chunk-major [ceil(ft_out/256)][rows][256]
-template <typename T>
-__global__ void to_chunk_major_kernel(const T* __restrict__ src, T* __restrict__ dst, uint64_t rows,
-                                      uint32_t ft_out) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * ft_out) return;
-    const uint64_t r = i / ft_out;
-    const uint32_t c = (uint32_t)(i - r * ft_out);
-    dst[(uint64_t)(c / kDftChunk) * rows * kDftChunk + r * kDftChunk + c % kDftChunk] = src[i];
+// Several buffers in one allocation, 256-byte aligned: an hipMalloc and an
+// hipFree cost about 8 us a pair, more for large ones.
+struct DevCarve {
+    DevScratch mem;
+    size_t bytes = 0;
+    // the buffer's offset; take(offset) after alloc()
+    size_t add(size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    }
+    int32_t alloc() { return mem.alloc(bytes); }
+    template <class T>
+    T* take(size_t at) {
+        return reinterpret_cast<T*>(mem.as<uint8_t>() + at);
+    }
+};
+
+// The occurrence lists of a batch, in one allocation.
+struct OccurrenceLists {
+    DevCarve ws;
+    uint32_t *vals = nullptr, *offsets = nullptr;
+    int32_t sort(const int32_t* stm_idx, const int32_t* nstm_idx, const int32_t* nnz, uint32_t batch,
+                 uint32_t max_active, uint32_t cols) {
+        const uint64_t n_items = 2ull * batch * max_active;
+        const size_t tb = occurrence_sort_temp_bytes(n_items, cols);
+        const size_t ki = ws.add(4 * n_items), vi = ws.add(4 * n_items), ko = ws.add(4 * n_items),
+                     vo = ws.add(4 * n_items), off = ws.add(4ull * (2ull * cols + 2)), tmp = ws.add(tb);
+        int32_t st = ws.alloc();
+        if (st) return st;
+        OccurrenceSortArgs os{};
+        os.idx_stm = stm_idx;
+        os.idx_nstm = nstm_idx;
+        os.nnz = nnz;
+        os.batch = batch;
+        os.max_active = max_active;
+        os.cols = cols;
+        os.keys_in = ws.take<uint32_t>(ki);
+        os.vals_in = ws.take<uint32_t>(vi);
+        os.keys_out = ws.take<uint32_t>(ko);
+        os.vals_out = vals = ws.take<uint32_t>(vo);
+        os.offsets = offsets = ws.take<uint32_t>(off);
+        os.temp = ws.take<uint8_t>(tmp);
+        os.temp_bytes = tb;
+        return launch_occurrence_sort(os, 0);
+    }
+};
+
+// row-major [rows][ft_out] -> chunk-major [ceil(ft_out/256)][rows][256], a V (of
+// row_v in a row and chunk_v in a chunk's row) a lane
+template <typename V>
+__global__ __launch_bounds__(256) void to_chunk_major_kernel(const V* __restrict__ src, V* __restrict__ dst,
+                                                             uint64_t rows, uint32_t row_v, uint32_t chunk_v) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= rows * row_v) return;
+    const uint64_t r = i / row_v;
+    const uint32_t c = (uint32_t)(i - r * row_v);
+    dst[(uint64_t)(c / chunk_v) * rows * chunk_v + r * chunk_v + c % chunk_v] = src[i];
 }
 
 __global__ void copy_f4_kernel(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n4) {
@@ -201,32 +251,32 @@ int32_t tatara_op_ft_forward_pairwise(const float* weight, const int32_t* stm_id
                                       uint32_t cols, uint32_t max_active, uint32_t piece_inputs,
                                       float scale) {
     TATARA_REQUIRE(ft_out % 8 == 0, "ft_out must be a multiple of 8");
-    DevScratch keys, sched, hist, bstart, bcount;
+    DevCarve ws;
     int32_t* schedule = nullptr;
     if (piece_inputs > 0 && batch > 0) {
         uint32_t n_bins = ceil_div(cols, piece_inputs);
         if (n_bins > 128) n_bins = 128;
         int32_t st;
-        if ((st = keys.alloc(2ull * batch)) || (st = sched.alloc(8ull * batch)) ||
-            (st = hist.alloc(4ull * 2 * n_bins * binsort_tiles(2 * batch))) ||
-            (st = bstart.alloc(4ull * (2 * n_bins + 1))) || (st = bcount.alloc(4ull * 2 * n_bins)))
-            return st;
-        st = launch_king_block_keys(stm_idx, nstm_idx, nnz, keys.as<uint8_t>(), batch, max_active,
+        const size_t keys = ws.add(2ull * batch), sched = ws.add(8ull * batch),
+                     hist = ws.add(4ull * 2 * n_bins * binsort_tiles(2 * batch)),
+                     bstart = ws.add(4ull * (2 * n_bins + 1)), bcount = ws.add(4ull * 2 * n_bins);
+        if ((st = ws.alloc())) return st;
+        st = launch_king_block_keys(stm_idx, nstm_idx, nnz, ws.take<uint8_t>(keys), batch, max_active,
                                     cols, piece_inputs, n_bins, 0);
         if (st) return st;
         BinSortArgs bs{};
-        bs.keys = keys.as<uint8_t>();
+        bs.keys = ws.take<uint8_t>(keys);
         bs.n_items = 2 * batch;
         bs.n_bins = 2 * n_bins;
         bs.align = 1;
         bs.value_mod = batch;
-        bs.hist = hist.as<uint32_t>();
-        bs.bin_start = bstart.as<uint32_t>();
-        bs.bin_count = bcount.as<uint32_t>();
-        bs.out = sched.as<int32_t>();
+        bs.hist = ws.take<uint32_t>(hist);
+        bs.bin_start = ws.take<uint32_t>(bstart);
+        bs.bin_count = ws.take<uint32_t>(bcount);
+        bs.out = ws.take<int32_t>(sched);
         st = launch_binsort(bs, 0);
         if (st) return st;
-        schedule = sched.as<int32_t>();
+        schedule = ws.take<int32_t>(sched);
     }
     FtForwardArgs a{};
     a.mode = 1;
@@ -257,35 +307,15 @@ int32_t tatara_op_ft_weight_grad(const float* dft, const int32_t* stm_idx,
                                  uint32_t max_active) {
     TATARA_REQUIRE(ft_out % 4 == 0, "ft_out must be a multiple of 4");
     TATARA_REQUIRE(max_active <= 64, "max_active must be <= 64");
-    const uint64_t n_items = 2ull * batch * max_active;
-    const uint32_t n_keys = 2 * cols + 1;
-    DevScratch ki, vi, ko, vo, off, tmp;
-    const size_t tb = occurrence_sort_temp_bytes(n_items, cols);
+    OccurrenceLists occ;
     int32_t st;
-    if ((st = ki.alloc(4 * n_items)) || (st = vi.alloc(4 * n_items)) || (st = ko.alloc(4 * n_items)) ||
-        (st = vo.alloc(4 * n_items)) || (st = off.alloc(4ull * (n_keys + 1))) || (st = tmp.alloc(tb)))
-        return st;
-    OccurrenceSortArgs os{};
-    os.idx_stm = stm_idx;
-    os.idx_nstm = nstm_idx;
-    os.nnz = nnz;
-    os.batch = batch;
-    os.max_active = max_active;
-    os.cols = cols;
-    os.keys_in = ki.as<uint32_t>();
-    os.vals_in = vi.as<uint32_t>();
-    os.keys_out = ko.as<uint32_t>();
-    os.vals_out = vo.as<uint32_t>();
-    os.offsets = off.as<uint32_t>();
-    os.temp = tmp.p;
-    os.temp_bytes = tb;
-    if ((st = launch_occurrence_sort(os, 0))) return st;
+    if ((st = occ.sort(stm_idx, nstm_idx, nnz, batch, max_active, cols))) return st;
     FtGradArgs g{};
     g.dft = dft;
     g.dft_row_stride = ft_out;  // row-major [2][batch][ft_out]
     g.dft_chunk_stride = kDftChunk;
-    g.occ_vals = vo.as<uint32_t>();
-    g.occ_off = off.as<uint32_t>();
+    g.occ_vals = occ.vals;
+    g.occ_off = occ.offsets;
     g.grad = grad;
     g.ft_out = ft_out;
     g.rows = cols;
@@ -307,47 +337,59 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
     uint32_t n_blocks = ceil_div(cols, piece_inputs);
     if (n_blocks > 128) n_blocks = 128;
     const uint64_t two_b = 2ull * batch;
-    const uint32_t chunks = ceil_div(ft_out, kDftChunk);
+    // a row-major dft of whole column chunks, four values aligned, is read where
+    // it lies; else its rows are laid out in chunks first (a value a lane where
+    // four are not aligned)
+    const uint64_t elem = dft16 ? 2 : 4;
+    const void* src = dft16 ? static_cast<const void*>(dft16) : static_cast<const void*>(dft);
+    const bool aligned = reinterpret_cast<uintptr_t>(src) % (4 * elem) == 0;
+    const bool in_place = aligned && ft_out % kDftChunk == 0;
+    const uint64_t chunk_bytes = in_place ? 0 : elem * ceil_div(ft_out, kDftChunk) * two_b * kDftChunk;
     // king-block schedule, as the trainer builds it for the forward
-    DevScratch keys, sched, hist, start, count, cm, multi, srows, smasks;
+    DevCarve ws;
     const uint64_t stages = ft_scan_max_stages(batch, n_blocks);
-    if ((st = keys.alloc(two_b)) || (st = sched.alloc(4 * two_b)) ||
-        (st = hist.alloc(4ull * 2 * n_blocks * binsort_tiles((uint32_t)two_b))) ||
-        (st = start.alloc(4ull * (2 * n_blocks + 1))) || (st = count.alloc(4ull * 2 * n_blocks)) ||
-        (st = cm.alloc(4ull * chunks * two_b * kDftChunk)) ||
-        (st = multi.alloc(4)) || (st = srows.alloc(4ull * stages * 32)) ||
-        (st = smasks.alloc(4ull * stages * ft_scan_mask_words(piece_inputs) * 16)))
-        return st;
-    if ((st = launch_king_block_keys(stm_idx, nstm_idx, nnz, keys.as<uint8_t>(), batch, max_active, cols,
+    const size_t keys = ws.add(two_b), sched = ws.add(4 * two_b),
+                 hist = ws.add(4ull * 2 * n_blocks * binsort_tiles((uint32_t)two_b)),
+                 start = ws.add(4ull * (2 * n_blocks + 1)), count = ws.add(4ull * 2 * n_blocks),
+                 multi = ws.add(4), srows = ws.add(4ull * stages * 32),
+                 smasks = ws.add(4ull * stages * ft_scan_mask_words(piece_inputs) * 16), cm = ws.add(chunk_bytes);
+    if ((st = ws.alloc())) return st;
+    if ((st = launch_king_block_keys(stm_idx, nstm_idx, nnz, ws.take<uint8_t>(keys), batch, max_active, cols,
                                      piece_inputs, n_blocks, 0)))
         return st;
     BinSortArgs bs{};
-    bs.keys = keys.as<uint8_t>();
+    bs.keys = ws.take<uint8_t>(keys);
     bs.n_items = (uint32_t)two_b;
     bs.n_bins = 2 * n_blocks;
     bs.align = 1;
     bs.value_mod = batch;
-    bs.hist = hist.as<uint32_t>();
-    bs.bin_start = start.as<uint32_t>();
-    bs.bin_count = count.as<uint32_t>();
-    bs.out = sched.as<int32_t>();
+    bs.hist = ws.take<uint32_t>(hist);
+    bs.bin_start = ws.take<uint32_t>(start);
+    bs.bin_count = ws.take<uint32_t>(count);
+    bs.out = ws.take<int32_t>(sched);
     if ((st = launch_binsort(bs, 0))) return st;
-    if (two_b * ft_out > 0) {
+    if (!in_place && two_b * ft_out > 0) {
+        const uint32_t per = aligned ? 4 : 1, row_v = ft_out / per, chunk_v = kDftChunk / per;
+        const uint32_t blocks = ceil_div(two_b * row_v, 256);
+        auto copy = [&](auto* zero) {
+            using V = std::remove_pointer_t<decltype(zero)>;
+            to_chunk_major_kernel<V><<<blocks, 256>>>(static_cast<const V*>(src), ws.take<V>(cm), two_b, row_v, chunk_v);
+        };
         if (dft16)
-            to_chunk_major_kernel<<<ceil_div(two_b * ft_out, 256), 256>>>(dft16, cm.as<uint16_t>(), two_b, ft_out);
+            aligned ? copy(static_cast<ushort4*>(nullptr)) : copy(static_cast<uint16_t*>(nullptr));
         else
-            to_chunk_major_kernel<<<ceil_div(two_b * ft_out, 256), 256>>>(dft, cm.as<float>(), two_b, ft_out);
+            aligned ? copy(static_cast<float4*>(nullptr)) : copy(static_cast<float*>(nullptr));
         TATARA_LAUNCHED("to_chunk_major");
     }
     FtBlockScan sc{};
     sc.idx_stm = stm_idx;
     sc.idx_nstm = nstm_idx;
     sc.nnz = nnz;
-    sc.schedule = sched.as<int32_t>();
-    sc.sched_start = start.as<uint32_t>();
-    sc.multi = multi.as<uint32_t>();
-    sc.stage_rows = srows.as<uint32_t>();
-    sc.stage_masks = smasks.as<uint32_t>();
+    sc.schedule = ws.take<int32_t>(sched);
+    sc.sched_start = ws.take<uint32_t>(start);
+    sc.multi = ws.take<uint32_t>(multi);
+    sc.stage_rows = ws.take<uint32_t>(srows);
+    sc.stage_masks = ws.take<uint32_t>(smasks);
     sc.batch = batch;
     sc.max_active = max_active;
     sc.cols = cols;
@@ -355,47 +397,31 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
     sc.n_blocks = n_blocks;
     sc.dealt = mfma ? 0u : 1u;
     if ((st = launch_ft_scan_tables(sc, 0))) return st;
-    // occurrence lists for the fallback (a row with features of two blocks)
-    const uint64_t n_items = two_b * max_active;
-    const uint32_t n_keys = 2 * cols + 1;
-    DevScratch ki, vi, ko, vo, off, tmp;
-    const size_t tb = occurrence_sort_temp_bytes(n_items, cols);
-    if ((st = ki.alloc(4 * n_items)) || (st = vi.alloc(4 * n_items)) || (st = ko.alloc(4 * n_items)) ||
-        (st = vo.alloc(4 * n_items)) || (st = off.alloc(4ull * (n_keys + 1))) || (st = tmp.alloc(tb)))
-        return st;
-    OccurrenceSortArgs os{};
-    os.idx_stm = stm_idx;
-    os.idx_nstm = nstm_idx;
-    os.nnz = nnz;
-    os.batch = batch;
-    os.max_active = max_active;
-    os.cols = cols;
-    os.keys_in = ki.as<uint32_t>();
-    os.vals_in = vi.as<uint32_t>();
-    os.keys_out = ko.as<uint32_t>();
-    os.vals_out = vo.as<uint32_t>();
-    os.offsets = off.as<uint32_t>();
-    os.temp = tmp.p;
-    os.temp_bytes = tb;
-    if ((st = launch_occurrence_sort(os, 0))) return st;
     FtGradArgs g{};
     if (dft16) {
-        g.dft16 = cm.as<uint16_t>();
+        g.dft16 = in_place ? dft16 : ws.take<uint16_t>(cm);
         g.dft_inv_scale = inv_scale;
     } else {
-        g.dft = cm.as<float>();
+        g.dft = in_place ? dft : ws.take<float>(cm);
     }
-    g.dft_row_stride = kDftChunk;
-    g.dft_chunk_stride = two_b * kDftChunk;
-    g.occ_vals = vo.as<uint32_t>();
-    g.occ_off = off.as<uint32_t>();
+    g.dft_row_stride = in_place ? ft_out : kDftChunk;
+    g.dft_chunk_stride = in_place ? kDftChunk : two_b * kDftChunk;
     g.grad = grad;
     g.ft_out = ft_out;
     g.rows = cols;
     g.apply_update = 0;
-    if ((st = mfma ? launch_ft_grad_mfma(g, sc, 0) : launch_ft_grad_scan(g, sc, 0))) return st;
+    // (does nothing when the tables found a row the scan cannot take)
+    if ((st = mfma ? launch_ft_grad_mfma(g, sc, 0, false) : launch_ft_grad_scan(g, sc, 0, false))) return st;
     uint32_t m = 0;
-    TATARA_HIP(hipMemcpy(&m, multi.p, 4, hipMemcpyDeviceToHost), "ft_weight_grad_blocked");
+    TATARA_HIP(hipMemcpy(&m, sc.multi, 4, hipMemcpyDeviceToHost), "ft_weight_grad_blocked");
+    if (m) {  // a row with features of two blocks, or one twice: occurrence lists
+        OccurrenceLists occ;
+        if ((st = occ.sort(stm_idx, nstm_idx, nnz, batch, max_active, cols))) return st;
+        g.occ_vals = occ.vals;
+        g.occ_off = occ.offsets;
+        if ((st = launch_ft_grad_update(g, 0))) return st;
+        TATARA_HIP(hipDeviceSynchronize(), "ft_weight_grad_blocked lists");
+    }
     if (used_block_scan) *used_block_scan = m ? 0u : 1u;
     return kOk;
 }
