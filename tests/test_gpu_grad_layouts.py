@@ -70,3 +70,29 @@ def test_f16_layouts_agree(gpu, b, ft_out):
             assert np.abs(got - exact * np.float32(inv)).max() <= (2 * b) ** 2 * 64 * 2.0 ** -24 * inv + 1e-30
             first = got if first is None else first
             assert np.array_equal(got, first), shift
+
+
+def test_kept_scratch_grows_and_is_each_threads_own(gpu):
+    """Calls of growing, shrinking and fallback sizes from three threads at once."""
+    import threading
+
+    def work(seed, bad):
+        try:
+            for b, ft_out, fallback in ((5, 256, False), (300, 260, False), (40, 512, True), (700, 768, False)):
+                b += seed
+                idx = rows(b, fallback)
+                dft = np.random.default_rng(b).normal(0, 1, (2, b, ft_out)).astype(np.float32)
+                want = _oracle_grad(dft, *idx, b, ft_out, KB * PI, MA).reshape(KB * PI, ft_out)
+                got, used = run(gpu, gpu.tatara_op_ft_weight_grad_blocked, dft, idx, b, ft_out, 0)
+                if used != (0 if fallback else 1) or not np.array_equal(got, want):
+                    bad.append((seed, b))
+        except Exception as e:
+            bad.append(repr(e))
+
+    bad = []
+    threads = [threading.Thread(target=work, args=(k, bad)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
