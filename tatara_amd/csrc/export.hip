@@ -39,28 +39,27 @@ constexpr uint64_t kQStep = (uint64_t)kQThreads * kQVec;           // values per
 constexpr uint64_t kQTile = kQStep * kQSteps;                      // values per workgroup
 constexpr int kScanThreads = 1024;
 
-// Row, column and virtual-row index of cell i.  32-bit division whenever the
+// Virtual row and column of cell i.  32-bit division whenever the
 // table has < 2^32 cells (every feature set at every supported width).
-__device__ __forceinline__ uint64_t virtual_offset(const QuantSource& s, uint64_t i) {
-    uint64_t c, p;
+struct VirtualCell {
+    uint32_t p, c;  // virtual row, column
+    __device__ __forceinline__ uint64_t at(const QuantSource& s) const { return (s.rows + p) * s.cols + c; }
+};
+__device__ __forceinline__ VirtualCell virtual_cell(const QuantSource& s, uint64_t i) {
     if (s.rows * s.cols < (1ull << 32)) {
         const uint32_t i32 = (uint32_t)i;
         const uint32_t r32 = i32 / s.cols;
-        c = i32 - r32 * s.cols;
-        p = r32 % s.piece_inputs;
-    } else {
-        const uint64_t r = i / s.cols;
-        c = i - r * s.cols;
-        p = r % s.piece_inputs;
+        return {r32 % s.piece_inputs, i32 - r32 * s.cols};
     }
-    return (s.rows + p) * s.cols + c;
+    const uint64_t r = i / s.cols;
+    return {(uint32_t)(r % s.piece_inputs), (uint32_t)(i - r * s.cols)};
 }
 
 // Cell i of the export-shape table: the real row's value plus, with a
 // factorizer, its piece's virtual row (an f32 add, as the fold does).
 __device__ __forceinline__ float source_value(const QuantSource& s, uint64_t i) {
     float v = s.w[i];
-    if (s.piece_inputs) v += s.w[virtual_offset(s, i)];
+    if (s.piece_inputs) v += s.w[virtual_cell(s, i).at(s)];
     return v;
 }
 
@@ -78,10 +77,22 @@ __device__ __forceinline__ void load_tile(const QuantSource& s, uint64_t n, uint
 #pragma unroll
         for (int k = 0; k < kQSteps; ++k) v[k] = *reinterpret_cast<const float4*>(s.w + t0 + k * kQStep);
         if (s.piece_inputs) {
+            // one division per thread: a step moves kQStep / cols rows on, and
+            // one more where the column passes the row's end
             float4 g[kQSteps];
+            VirtualCell vc = virtual_cell(s, t0);
+            const uint32_t dr = (uint32_t)kQStep / s.cols % s.piece_inputs, dc = (uint32_t)kQStep % s.cols;
 #pragma unroll
-            for (int k = 0; k < kQSteps; ++k)
-                g[k] = *reinterpret_cast<const float4*>(s.w + virtual_offset(s, t0 + k * kQStep));
+            for (int k = 0; k < kQSteps; ++k) {
+                g[k] = *reinterpret_cast<const float4*>(s.w + vc.at(s));
+                vc.c += dc;
+                vc.p += dr;
+                if (vc.c >= s.cols) {
+                    vc.c -= s.cols;
+                    ++vc.p;
+                }
+                if (vc.p >= s.piece_inputs) vc.p -= s.piece_inputs;
+            }
 #pragma unroll
             for (int k = 0; k < kQSteps; ++k) {
                 v[k].x += g[k].x;
@@ -106,17 +117,23 @@ __device__ __forceinline__ void load_tile(const QuantSource& s, uint64_t n, uint
         }
 }
 
-// saturate_i16(round(scale * v)) with NaN -> 0.
+// saturate_i16(round(scale * v)) with NaN -> 0.  Half away from zero: the
+// truncation of x + copysign(h, x) with h the double below 0.5, which takes every
+// k + 0.5 to k + 1 and no value below k + 0.5 there; v_cvt_i32_f64 truncates,
+// saturates and sends NaN to 0 (six instructions; round() and the comparisons
+// on doubles were the larger part of the kernels' instructions).
 __device__ __forceinline__ int32_t quant16(float v, double scale) {
     const double x = scale * (double)v;
-    if (x != x) return 0;
-    const double r = round(x);
-    return r < -32768.0 ? -32768 : (r > 32767.0 ? 32767 : (int32_t)r);
+    const double y = x + copysign(0x1.fffffffffffffp-2, x);
+    int32_t q;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(q) : "v"(y));
+    return min(max(q, -32768), 32767);
 }
 
 // Signed LEB128 length of an i16 value.
 __device__ __forceinline__ uint32_t leb128_len(int32_t q) {
-    return (q >= -64 && q < 64) ? 1u : ((q >= -8192 && q < 8192) ? 2u : 3u);
+    const uint32_t u = (uint32_t)(q ^ (q >> 31));  // one's-complement magnitude
+    return 1u + (u >= 64u) + (u >= 8192u);
 }
 
 __global__ __launch_bounds__(256) void quantise_i16_kernel(QuantSource s, double scale, uint64_t n,
@@ -126,7 +143,16 @@ __global__ __launch_bounds__(256) void quantise_i16_kernel(QuantSource s, double
         out[i] = (int16_t)quant16(source_value(s, i), scale);
 }
 
-// Pass 1: bytes of each tile of kQTile values.
+// leb128_len(quant16(v, scale)) without the rounding: round (half away) is
+// >= 64 from 63.5 up and <= -65 from -64.5 down; NaN is 0 and takes one byte.
+__device__ __forceinline__ uint32_t quant_len(float v, double scale) {
+    const double x = scale * (double)v;
+    return (x >= 63.5 || x <= -64.5) ? ((x >= 8191.5 || x <= -8192.5) ? 3u : 2u) : 1u;
+}
+
+// Pass 1: bytes of each tile of kQTile values.  A read of the table (450 MB at
+// ft_out 1536 135 -> 125 us, 3.6 TB/s); run once per stream, its offsets serve
+// the capacity check and pass 3.
 __global__ __launch_bounds__(kQThreads) void leb128_tile_bytes_kernel(QuantSource s, double scale, uint64_t n,
                                                                       uint32_t* __restrict__ tile_bytes) {
     const uint64_t base = (uint64_t)blockIdx.x * kQTile;
@@ -138,78 +164,143 @@ __global__ __launch_bounds__(kQThreads) void leb128_tile_bytes_kernel(QuantSourc
     for (int k = 0; k < kQSteps; ++k)
 #pragma unroll
         for (int j = 0; j < kQVec; ++j)
-            if (t0 + k * kQStep + j < n) sum += leb128_len(quant16(x[k][j], scale));
+            if (t0 + k * kQStep + j < n) sum += quant_len(x[k][j], scale);
     using Reduce = hipcub::BlockReduce<uint32_t, kQThreads>;
     __shared__ typename Reduce::TempStorage tmp;
     const uint32_t total = Reduce(tmp).Sum(sum);
     if (threadIdx.x == 0) tile_bytes[blockIdx.x] = total;
 }
 
-// Pass 2: exclusive offsets of the tiles (one workgroup; each thread owns a
-// contiguous run of tiles) and the stream's total length.
+// Pass 2: exclusive offsets of the tiles and the stream's total length.  A
+// workgroup for every 1024 tiles; each sums the counts before its own by itself
+// (110 KB at most are read again at 27,489 tiles) instead of waiting for the
+// workgroup before it.  One workgroup over all tiles, each thread a contiguous
+// run, one load after another: 46 us, now 7 us.
 __global__ __launch_bounds__(kScanThreads) void leb128_tile_scan_kernel(const uint32_t* __restrict__ tile_bytes,
                                                                         uint64_t n_tiles,
                                                                         uint64_t* __restrict__ tile_off,
                                                                         uint64_t* __restrict__ total) {
-    const uint64_t per = (n_tiles + kScanThreads - 1) / kScanThreads;
-    const uint64_t a = min(n_tiles, (uint64_t)threadIdx.x * per);
-    const uint64_t b = min(n_tiles, a + per);
-    uint64_t run = 0;
-    for (uint64_t i = a; i < b; ++i) run += tile_bytes[i];
-    using Scan = hipcub::BlockScan<uint64_t, kScanThreads>;
-    __shared__ typename Scan::TempStorage tmp;
-    uint64_t excl, agg;
-    Scan(tmp).ExclusiveSum(run, excl, agg);
-    for (uint64_t i = a; i < b; ++i) {
-        tile_off[i] = excl;
-        excl += tile_bytes[i];
+    constexpr uint32_t kWaves = kScanThreads / 64;
+    __shared__ uint64_t s_before[kWaves], s_own[kWaves];
+    const uint32_t t = threadIdx.x, lane = t % 64, wave = t / 64;
+    const uint64_t base = (uint64_t)blockIdx.x * kScanThreads, i = base + t;
+    const uint32_t v = i < n_tiles ? tile_bytes[i] : 0u;
+    uint64_t before = 0;
+    uint64_t k = t;
+    for (; k + 3 * kScanThreads < base; k += 4 * kScanThreads)
+        before += (uint64_t)tile_bytes[k] + tile_bytes[k + kScanThreads] + tile_bytes[k + 2 * kScanThreads] +
+                  tile_bytes[k + 3 * kScanThreads];
+    for (; k < base; k += kScanThreads) before += tile_bytes[k];
+    uint64_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t y = __shfl_up(incl, d);
+        if (lane >= (uint32_t)d) incl += y;
+        before += __shfl_xor(before, d);
     }
-    if (threadIdx.x == 0) *total = agg;
+    if (lane == 63) {
+        s_own[wave] = incl;
+        s_before[wave] = before;
+    }
+    __syncthreads();
+    uint64_t off = incl - v, all = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; ++w) {
+        off += s_before[w] + (w < wave ? s_own[w] : 0ull);
+        all += s_before[w] + s_own[w];
+    }
+    if (i < n_tiles) tile_off[i] = off;
+    if (blockIdx.x + 1 == gridDim.x && t == 0) *total = all;
 }
 
 // Pass 3: each tile re-quantises its values and writes their LEB128 bytes in
-// cell order: step by step, thread t's four cells follow threads 0..t-1's.
+// cell order: step by step, thread t's four cells follow threads 0..t-1's.  One
+// scan gives the offsets of all four steps (16-bit fields: a step's bytes are at
+// most 3072); the bytes are put together in LDS, placed so that its 16-byte
+// blocks lie on the output's, and leave as whole blocks, the first and last
+// byte by byte.  Stored from registers byte by byte, with a scan per step, the
+// pass took 193 us at ft_out 1536, now 163 us (450 MB read, 225 MB written: 4.1
+// TB/s, bound by memory; with round() and a division per four cells 242 us).  The
+// tiles go last to first: pass 1 has left the table's end in the last-level cache
+// (first to last 167 us).
 __global__ __launch_bounds__(kQThreads) void leb128_scatter_kernel(QuantSource s, double scale, uint64_t n,
                                                                    const uint64_t* __restrict__ tile_off,
                                                                    uint8_t* __restrict__ out) {
-    using Scan = hipcub::BlockScan<uint32_t, kQThreads>;
-    __shared__ typename Scan::TempStorage tmp;
-    const uint64_t base = (uint64_t)blockIdx.x * kQTile;
+    static_assert(kQSteps == 4 && kQVec == 4 && kQStep * 3 < 65536, "four 16-bit step lengths");
+    constexpr uint32_t kBlocks = (3 * kQTile + 15 + 15) / 16;  // 16-byte blocks the tile's bytes can touch
+    __shared__ __align__(16) uint32_t s_out[kBlocks * 4];
+    __shared__ uint64_t s_wave[kQThreads / 64];
+    const uint32_t t = threadIdx.x, lane = t % 64, wave = t / 64;
+    const uint32_t tile = gridDim.x - 1 - blockIdx.x;
+    const uint64_t base = (uint64_t)tile * kQTile;
     float x[kQSteps][kQVec];
     load_tile(s, n, base, x);
-    const uint64_t t0 = base + (uint64_t)kQVec * threadIdx.x;
-    uint64_t off = tile_off[blockIdx.x];
+    for (uint32_t i = t; i < kBlocks; i += kQThreads) reinterpret_cast<uint4*>(s_out)[i] = make_uint4(0, 0, 0, 0);
+    const uint64_t t0 = base + (uint64_t)kQVec * t;
+    uint64_t lo[kQSteps];  // a step's bytes, low first: 12 at most
+    uint32_t hi[kQSteps];
+    uint64_t lens = 0;
+#pragma unroll
     for (int k = 0; k < kQSteps; ++k) {
-        int32_t q[kQVec];
-        uint32_t len = 0;
+        uint32_t w[kQVec], l[kQVec];
 #pragma unroll
         for (int j = 0; j < kQVec; ++j) {
-            q[j] = quant16(x[k][j], scale);
-            if (t0 + k * kQStep + j < n) len += leb128_len(q[j]);
+            const uint32_t v = (uint32_t)quant16(x[k][j], scale);
+            l[j] = t0 + k * kQStep + j < n ? leb128_len((int32_t)v) : 0u;
+            // 7 bits a byte, the top bit of all but the last byte set
+            const uint32_t all = (v & 0x7fu) | (v << 1 & 0x7f00u) | (v << 2 & 0x7f0000u) | 0x8080u;
+            w[j] = all & ((1u << (8 * l[j])) - 1u) & ~(0x80u << (8 * l[j]) >> 8);
         }
-        uint32_t excl, agg;
-        Scan(tmp).ExclusiveSum(len, excl, agg);
-        uint8_t* p = out + off + excl;
-#pragma unroll
-        for (int j = 0; j < kQVec; ++j) {
-            if (t0 + k * kQStep + j >= n) break;
-            const int32_t v = q[j];
-            const uint32_t l = leb128_len(v);
-            if (l == 1) {
-                p[0] = (uint8_t)(v & 0x7f);
-            } else if (l == 2) {
-                p[0] = (uint8_t)((v & 0x7f) | 0x80);
-                p[1] = (uint8_t)((v >> 7) & 0x7f);
-            } else {
-                p[0] = (uint8_t)((v & 0x7f) | 0x80);
-                p[1] = (uint8_t)(((v >> 7) & 0x7f) | 0x80);
-                p[2] = (uint8_t)((v >> 14) & 0x7f);
-            }
-            p += l;
-        }
-        off += agg;
-        __syncthreads();  // the scan's temp storage is reused by the next step
+        const uint64_t p = w[0] | (uint64_t)w[1] << (8 * l[0]);  // 6 bytes at most
+        const uint64_t q = w[2] | (uint64_t)w[3] << (8 * l[2]);
+        const uint32_t lp = l[0] + l[1];
+        lo[k] = p | q << (8 * lp);
+        hi[k] = (uint32_t)(q >> 16 >> (48 - 8 * lp));  // lp <= 6; none when lp is 0 (q is then 0 too)
+        lens |= (uint64_t)(lp + l[2] + l[3]) << (16 * k);
     }
+    // inclusive scan of the four fields over the workgroup
+    uint64_t incl = lens;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t y = __shfl_up(incl, d);
+        if (lane >= (uint32_t)d) incl += y;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();  // s_wave, s_out zeroed
+    uint64_t before = incl - lens, all = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kQThreads / 64; ++w) {
+        before += w < wave ? s_wave[w] : 0ull;
+        all += s_wave[w];
+    }
+    uint8_t* dst = out + tile_off[tile];
+    const uint32_t lead = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u);  // the tile's place in its first block
+    uint32_t step0 = lead;
+#pragma unroll
+    for (int k = 0; k < kQSteps; ++k) {
+        const uint32_t at = step0 + (uint32_t)(before >> (16 * k) & 0xffffu);
+        const uint32_t len = (uint32_t)(lens >> (16 * k) & 0xffffu);
+        const uint32_t sh = 8 * (at & 3u), word = at >> 2, end = (at + len + 3) >> 2;
+        // the 96 bits shifted up to the byte, in four words
+        const uint64_t a0 = lo[k] << sh;
+        const uint64_t a1 = ((uint64_t)hi[k] << sh) | (sh ? lo[k] >> (64 - sh) : 0ull);
+        if (word < end) atomicOr(&s_out[word], (uint32_t)a0);
+        if (word + 1 < end) atomicOr(&s_out[word + 1], (uint32_t)(a0 >> 32));
+        if (word + 2 < end) atomicOr(&s_out[word + 2], (uint32_t)a1);
+        if (word + 3 < end) atomicOr(&s_out[word + 3], (uint32_t)(a1 >> 32));
+        step0 += (uint32_t)(all >> (16 * k) & 0xffffu);
+    }
+    __syncthreads();
+    // bytes [lead, step0) of the blocks
+    const uint8_t* s_bytes = reinterpret_cast<const uint8_t*>(s_out);
+    uint8_t* blocks = dst - lead;
+    const uint32_t first = (lead + 15) / 16, last = step0 / 16;  // whole blocks
+    for (uint32_t i = first + t; i < last; i += kQThreads)
+        reinterpret_cast<uint4*>(blocks)[i] = reinterpret_cast<const uint4*>(s_out)[i];
+    const uint32_t head = first <= last ? 16 * first : step0;  // bytes before the first whole block
+    if (t < 16 && lead + t < head && lead + t < step0) blocks[lead + t] = s_bytes[lead + t];
+    if (t >= 64 && t < 80 && first <= last && 16 * last + (t - 64) < step0 && 16 * last + (t - 64) >= head)
+        blocks[16 * last + (t - 64)] = s_bytes[16 * last + (t - 64)];
 }
 
 inline uint32_t ceil_div_u32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
@@ -313,8 +404,8 @@ int32_t launch_quantise_i16(const QuantSource& s, double scale, int16_t* out, hi
     return kOk;
 }
 
-int32_t launch_quantise_leb128(const QuantSource& s, double scale, uint32_t* tile_bytes, uint64_t* tile_off,
-                               uint64_t* d_total, uint8_t* out, hipStream_t stream) {
+int32_t launch_leb128_offsets(const QuantSource& s, double scale, uint32_t* tile_bytes, uint64_t* tile_off,
+                              uint64_t* d_total, hipStream_t stream) {
     const uint64_t n = s.rows * s.cols;
     const uint64_t tiles = leb128_tiles(n);
     TATARA_REQUIRE(tiles < (1ull << 31), "quantise: table too large");
@@ -322,12 +413,20 @@ int32_t launch_quantise_leb128(const QuantSource& s, double scale, uint32_t* til
         leb128_tile_bytes_kernel<<<(uint32_t)tiles, kQThreads, 0, stream>>>(s, scale, n, tile_bytes);
         TATARA_LAUNCHED("leb128_tile_bytes");
     }
-    leb128_tile_scan_kernel<<<1, kScanThreads, 0, stream>>>(tile_bytes, tiles, tile_off, d_total);
+    const uint32_t scans = tiles ? (uint32_t)((tiles + kScanThreads - 1) / kScanThreads) : 1u;
+    leb128_tile_scan_kernel<<<scans, kScanThreads, 0, stream>>>(tile_bytes, tiles, tile_off, d_total);
     TATARA_LAUNCHED("leb128_tile_scan");
-    if (tiles && out) {
-        leb128_scatter_kernel<<<(uint32_t)tiles, kQThreads, 0, stream>>>(s, scale, n, tile_off, out);
-        TATARA_LAUNCHED("leb128_scatter");
-    }
+    return kOk;
+}
+
+int32_t launch_leb128_scatter(const QuantSource& s, double scale, const uint64_t* tile_off, uint8_t* out,
+                              hipStream_t stream) {
+    const uint64_t n = s.rows * s.cols;
+    const uint64_t tiles = leb128_tiles(n);
+    TATARA_REQUIRE(tiles < (1ull << 31), "quantise: table too large");
+    if (tiles == 0) return kOk;
+    leb128_scatter_kernel<<<(uint32_t)tiles, kQThreads, 0, stream>>>(s, scale, n, tile_off, out);
+    TATARA_LAUNCHED("leb128_scatter");
     return kOk;
 }
 
@@ -370,16 +469,15 @@ int32_t quantise_leb128_to_host(const QuantSource& s, double scale, HostBytes& o
     hipError_t e = hipMalloc(&tile_bytes, (tiles + 1) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&tile_off, (tiles + 1) * sizeof(uint64_t));
     uint64_t bytes = 0;
-    if (e == hipSuccess) st = launch_quantise_leb128(s, scale, tile_bytes, tile_off, tile_off + tiles, nullptr, stream);
+    if (e == hipSuccess) st = launch_leb128_offsets(s, scale, tile_bytes, tile_off, tile_off + tiles, stream);
     if (e == hipSuccess && st == kOk)
         e = hipMemcpyAsync(&bytes, tile_off + tiles, sizeof bytes, hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess && st == kOk) e = hipStreamSynchronize(stream);
     if (e == hipSuccess && st == kOk) st = out.alloc(bytes);
     if (e == hipSuccess && st == kOk && bytes) e = hipMalloc(&d, bytes);
+    if (e == hipSuccess && st == kOk && bytes) st = launch_leb128_scatter(s, scale, tile_off, d, stream);
     if (e == hipSuccess && st == kOk && bytes) {
-        leb128_scatter_kernel<<<(uint32_t)tiles, kQThreads, 0, stream>>>(s, scale, n, tile_off, d);
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(out.p, d, bytes, hipMemcpyDeviceToHost, stream);
+        e = hipMemcpyAsync(out.p, d, bytes, hipMemcpyDeviceToHost, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
     (void)hipFree(d);

@@ -26,13 +26,16 @@ struct QuantSource {
     uint32_t piece_inputs = 0;  // 0: no virtual rows
 };
 
-// Device launchers.  quantise_leb128 needs `out` with room for 3 bytes per
-// value; the byte count lands in *d_total (device).  tile_bytes / tile_off
-// hold leb128_tiles(n) entries.
+// Device launchers.  The LEB128 stream comes in two steps, so that a caller can
+// check its length (*d_total, device) against the room it has before anything is
+// written: leb128_offsets counts, leb128_scatter writes *d_total bytes from the
+// same tile_off.  tile_bytes / tile_off hold leb128_tiles(n) entries.
 uint64_t leb128_tiles(uint64_t n);
 int32_t launch_quantise_i16(const QuantSource& s, double scale, int16_t* out, hipStream_t stream);
-int32_t launch_quantise_leb128(const QuantSource& s, double scale, uint32_t* tile_bytes, uint64_t* tile_off,
-                               uint64_t* d_total, uint8_t* out, hipStream_t stream);
+int32_t launch_leb128_offsets(const QuantSource& s, double scale, uint32_t* tile_bytes, uint64_t* tile_off,
+                              uint64_t* d_total, hipStream_t stream);
+int32_t launch_leb128_scatter(const QuantSource& s, double scale, const uint64_t* tile_off, uint8_t* out,
+                              hipStream_t stream);
 
 // Uninitialised host bytes, freed on destruction.  Ordinary pageable memory
 // on purpose: the file writer reads these bytes with the CPU, and CPU reads

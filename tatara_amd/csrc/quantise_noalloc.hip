@@ -1,7 +1,7 @@
 // FT-table quantisation without any device allocation.
 //
-// tatara_op_quantise_ft allocates the LEB128 path's per-tile byte counts and
-// offsets on every call.  Callers that cannot allocate device memory (code
+// tatara_op_quantise_ft may allocate the LEB128 path's per-tile byte counts and
+// offsets.  Callers that cannot allocate device memory (code
 // under HIP graph capture, tight serving loops, harnesses that forbid
 // hipMalloc) use tatara_op_quantise_ft_noalloc instead: the same kernels, with
 // those arrays in a file-scope device array of fixed size.  Each GPU the
@@ -84,12 +84,11 @@ int32_t tatara_op_quantise_ft_noalloc(const float* w, uint64_t rows, uint32_t co
     if (st) return st;
     uint64_t* tile_off = base;  // tile offsets, then the total in the last slot
     uint32_t* tile_bytes = reinterpret_cast<uint32_t*>(base + kOffWords);
-    if ((st = launch_quantise_leb128(src, scale, tile_bytes, tile_off, tile_off + tiles, nullptr, 0))) return st;
+    if ((st = launch_leb128_offsets(src, scale, tile_bytes, tile_off, tile_off + tiles, 0))) return st;
     uint64_t total = 0;
     TATARA_HIP(hipMemcpy(&total, tile_off + tiles, sizeof total, hipMemcpyDeviceToHost), "quantise_ft_noalloc total");
     TATARA_REQUIRE(total <= out_capacity, "out_capacity is smaller than the LEB128 stream");
-    if (total && (st = launch_quantise_leb128(src, scale, tile_bytes, tile_off, tile_off + tiles, out, 0)))
-        return st;
+    if (total && (st = launch_leb128_scatter(src, scale, tile_off, out, 0))) return st;
     TATARA_HIP(hipDeviceSynchronize(), "quantise_ft_noalloc");
     *out_bytes = total;
     return kOk;

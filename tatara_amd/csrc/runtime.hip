@@ -553,26 +553,18 @@ int32_t tatara_op_quantise_ft(const float* w, uint64_t rows, uint32_t cols, uint
         return kOk;
     }
     const uint64_t tiles = leb128_tiles(n);
-    uint32_t* tile_bytes = nullptr;
-    uint64_t* tile_off = nullptr;  // tile offsets, then the total in the last slot
-    TATARA_HIP(hipMalloc(&tile_bytes, (tiles + 1) * sizeof(uint32_t)), "hipMalloc quantise_ft");
-    hipError_t e = hipMalloc(&tile_off, (tiles + 1) * sizeof(uint64_t));
-    int32_t st = kOk;
+    DevCarve ws;  // tile byte counts; tile offsets, then the total in the last slot
+    const size_t counts = ws.add((tiles + 1) * sizeof(uint32_t)), offsets = ws.add((tiles + 1) * sizeof(uint64_t));
+    int32_t st;
+    if ((st = ws.alloc())) return st;
+    uint32_t* tile_bytes = ws.take<uint32_t>(counts);
+    uint64_t* tile_off = ws.take<uint64_t>(offsets);
+    if ((st = launch_leb128_offsets(src, scale, tile_bytes, tile_off, tile_off + tiles, 0))) return st;
     uint64_t total = 0;
-    if (e == hipSuccess) st = launch_quantise_leb128(src, scale, tile_bytes, tile_off, tile_off + tiles, nullptr, 0);
-    if (e == hipSuccess && st == kOk)
-        e = hipMemcpy(&total, tile_off + tiles, sizeof total, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && st == kOk && total > out_capacity) {
-        set_error("invalid argument: out_capacity is smaller than the LEB128 stream");
-        st = kErrInvalid;
-    }
-    if (e == hipSuccess && st == kOk && total)
-        st = launch_quantise_leb128(src, scale, tile_bytes, tile_off, tile_off + tiles, out, 0);
-    if (e == hipSuccess && st == kOk) e = hipDeviceSynchronize();
-    (void)hipFree(tile_off);
-    (void)hipFree(tile_bytes);
-    if (st) return st;
-    TATARA_HIP(e, "quantise_ft");
+    TATARA_HIP(hipMemcpy(&total, tile_off + tiles, sizeof total, hipMemcpyDeviceToHost), "quantise_ft total");
+    TATARA_REQUIRE(total <= out_capacity, "out_capacity is smaller than the LEB128 stream");
+    if (total && (st = launch_leb128_scatter(src, scale, tile_off, out, 0))) return st;
+    TATARA_HIP(hipDeviceSynchronize(), "quantise_ft");
     *out_bytes = total;
     return kOk;
 }
