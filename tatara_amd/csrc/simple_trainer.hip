@@ -448,11 +448,28 @@ class SimpleTrainer final : public TrainerBase {
         if ((st = forward(p, wdl_lambda, lp, 1, slot))) return st;
         const SimpleDenseArgs da = dense_args(p, wdl_lambda, lp, slot);
         if ((st = prof_mark(3))) return st;
-        if ((st = launch_simple_l1_weight_grad(da, stream))) return st;
+        if ((st = fork_dense())) return st;
+        if ((st = launch_simple_l1_weight_grad(da, dense_stream()))) return st;
         if ((st = launch_simple_l1_input_post(da, stream))) return st;
         if ((st = prof_mark(4))) return st;
 
         step_count += 1;
+        auto finalize_dense = [&]() -> int32_t {
+            SimpleDenseGroup groups[7];
+            for (int k = 0; k < 7; ++k) {
+                groups[k].w = small[k].w;
+                groups[k].m = small[k].m;
+                groups[k].v = small[k].v;
+                groups[k].slow = small[k].slow;
+                groups[k].grad = small[k].grad;
+                groups[k].n = small[k].n;
+                groups[k].min_w = small[k].min_w;
+                groups[k].max_w = small[k].max_w;
+                groups[k].kind = small[k].kind;
+            }
+            return launch_simple_dense_finalize(da, groups, scalars(1, lr, step_count),
+                                                   scalars(2, lr, step_count), cfg.keep_grads, dense_stream());
+        };
         FtGradArgs fb{};
         fb.dft = dft;
         fb.dft_row_stride = kDftChunk;  // chunk-major [chunk][2*b][256]
@@ -468,26 +485,12 @@ class SimpleTrainer final : public TrainerBase {
         fb.rows = ft_in;
         fb.apply_update = 1;
         fb.opt = scalars(0, lr, step_count);
-        if ((st = join_side())) return st;
+        if (!profiling && ((st = fork_side()) || (st = finalize_dense()))) return st;
         if ((st = ft_gradient(p, fb))) return st;
         if ((st = prof_mark(5))) return st;
         if (factorized && (st = launch_ft_virtual_fold(fb, pi, comb, nullptr, stream, table_layout()))) return st;
         if ((st = prof_mark(6))) return st;
-        SimpleDenseGroup groups[7];
-        for (int k = 0; k < 7; ++k) {
-            groups[k].w = small[k].w;
-            groups[k].m = small[k].m;
-            groups[k].v = small[k].v;
-            groups[k].slow = small[k].slow;
-            groups[k].grad = small[k].grad;
-            groups[k].n = small[k].n;
-            groups[k].min_w = small[k].min_w;
-            groups[k].max_w = small[k].max_w;
-            groups[k].kind = small[k].kind;
-        }
-        if ((st = launch_simple_dense_finalize(da, groups, scalars(1, lr, step_count),
-                                               scalars(2, lr, step_count), cfg.keep_grads, stream)))
-            return st;
+        if ((st = profiling ? finalize_dense() : join_side())) return st;
         if ((st = prof_mark(7))) return st;
         last_b = p.b;
         if ((st = release_batch())) return st;

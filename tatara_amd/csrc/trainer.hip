@@ -586,7 +586,8 @@ class LayerStackTrainer final : public TrainerBase {
         if ((st = forward(p, wdl_lambda, lp, 1, slot, padded))) return st;
         LsDenseArgs da = dense_args(p, padded, wdl_lambda, lp, slot);
         if ((st = prof_mark(3))) return st;
-        if ((st = launch_ls_l1_weight_grad(da, stream))) return st;
+        if ((st = fork_dense())) return st;
+        if ((st = launch_ls_l1_weight_grad(da, dense_stream()))) return st;
         if ((st = launch_ls_l1_input_post(da, stream))) return st;
         if ((st = prof_mark(4))) return st;
 
@@ -595,6 +596,21 @@ class LayerStackTrainer final : public TrainerBase {
         const OptScalars sf = scalars(0, lr, step_count);
         const OptScalars sd = scalars(1, lr, step_count);
         const OptScalars sb = scalars(2, lr, step_count);
+        auto finalize_dense = [&]() -> int32_t {
+            LsDenseGroup groups[9];
+            for (int k = 0; k < 9; ++k) {
+                groups[k].w = small[k].w;
+                groups[k].m = small[k].m;
+                groups[k].v = small[k].v;
+                groups[k].slow = small[k].slow;
+                groups[k].grad = small[k].grad;
+                groups[k].n = small[k].n;
+                groups[k].min_w = small[k].min_w;
+                groups[k].max_w = small[k].max_w;
+                groups[k].kind = small[k].kind;
+            }
+            return launch_ls_dense_finalize(da, groups, sd, sb, 1, cfg.keep_grads, dense_stream());
+        };
         FtGradArgs fb{};
         fb.dft = dft;
         fb.dft16 = dft16;
@@ -617,7 +633,7 @@ class LayerStackTrainer final : public TrainerBase {
         fb.rows = ft_in;
         fb.apply_update = 1;
         fb.opt = sf;
-        if ((st = join_side())) return st;
+        if (!profiling && ((st = fork_side()) || (st = finalize_dense()))) return st;
         if ((st = ft_gradient(p, fb))) return st;
         if ((st = prof_mark(5))) return st;
         if (factorized &&
@@ -625,19 +641,7 @@ class LayerStackTrainer final : public TrainerBase {
             return st;
         if (h_out) clamp_elems += 2ull * p.b * ft_out;
         if ((st = prof_mark(6))) return st;
-        LsDenseGroup groups[9];
-        for (int k = 0; k < 9; ++k) {
-            groups[k].w = small[k].w;
-            groups[k].m = small[k].m;
-            groups[k].v = small[k].v;
-            groups[k].slow = small[k].slow;
-            groups[k].grad = small[k].grad;
-            groups[k].n = small[k].n;
-            groups[k].min_w = small[k].min_w;
-            groups[k].max_w = small[k].max_w;
-            groups[k].kind = small[k].kind;
-        }
-        if ((st = launch_ls_dense_finalize(da, groups, sd, sb, 1, cfg.keep_grads, stream))) return st;
+        if ((st = profiling ? finalize_dense() : join_side())) return st;
         if ((st = prof_mark(7))) return st;
 
         // lagged loss (AsyncLossRing::read_and_queue_next)

@@ -178,6 +178,22 @@ class TrainerBase {
     int32_t fork_side();
     // stream waits for everything enqueued on side so far
     int32_t join_side();
+    // The dense weight gradients and their update run on the side stream, beside
+    // the input gradient and the feature-table gradient, which do not need them:
+    // five or six small launches, 50 to 60 us one after another that leave most of
+    // the chip idle, beside one of 150 us and more that memory bounds.  A step of
+    // Simple 256, batch 4096 449 -> 425 us, LayerStack 512 without factorizer,
+    // batch 2048 458 -> 445, LayerStack 768, batch 16384 1163 -> 1130; at 1536,
+    // batch 65536 both sides are bound by memory (4057 -> 4046).  While phases are
+    // profiled they stay on `stream`, so that each phase's time is its own.
+    // fork_dense: stream has what was queued on side before it, side what was
+    // queued on stream.
+    hipStream_t dense_stream() const { return profiling ? stream : side; }
+    int32_t fork_dense() {
+        int32_t st;
+        if ((st = join_side())) return st;
+        return profiling ? kOk : fork_side();
+    }
 };
 
 // The stream a trainer handle's steps run on (work enqueued there before a

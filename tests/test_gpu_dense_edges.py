@@ -53,3 +53,23 @@ def test_layerstack_edges(gpu, ft_out, l1, l2, b, factorize):
             gt.close(t.activation(name, b * ft_out), a[name], 1e-4, atol=1e-5 * top, what=name)
         for name in GROUPS:
             gt.close(t.get(name, "grad"), g[name], 1e-4, atol_frac=1e-5, what=f"grad {name}")
+
+
+@pytest.mark.parametrize("arch", ["simple", "layerstack", "unfactorized"])
+def test_dense_gradients_beside_the_table_gradient(gpu, arch):
+    """The dense side stream against the one stream of a profiled trainer: equal bits after four steps."""
+    b, out = 720, []
+    for profiled in (False, True):
+        if arch == "simple":
+            _, cfg = gs.make(ft_out=256, l1=32, l2=32, optimizer="adamw", b=b)
+            t, groups, args = SimpleTrainer(cfg), SIMPLE_GROUPS, (gs.batch_for(b, b),)
+        else:
+            sh, cfg = gt.make(ft_out=512, l1=16, l2=32, b=b, factorize=arch == "layerstack")
+            t, groups, args = LayerStackTrainer(cfg), GROUPS, gt.batch_for(b, b, sh.nb)
+        with t:
+            t.set_profiling(profiled)
+            losses = [t.train_step(*args, 1e-3, 0.25, Sigmoid()) for _ in range(4)]
+            losses.append(t.flush_pending_loss())
+            out.append([np.array(losses)] + [t.get(n, k) for n in groups for k in ("w", "m", "v")])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
