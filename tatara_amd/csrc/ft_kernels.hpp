@@ -108,7 +108,15 @@ struct FtGradArgs {
     int32_t apply_update;      // 0: only write gradients
     OptScalars opt;
     const uint32_t* run_if;    // when non-null the kernel does nothing unless *run_if != 0
+    // Block scan with a factorizer whose caller keeps no gradients (else null):
+    // [piece_inputs][kRowLiveStride], byte (p, K) says whether row K * pi + p has
+    // an occurrence in the batch.  The scan leaves the gradients of the other rows
+    // unwritten, and the fold takes them as zero.  Meaningless in a step whose
+    // *live_off is set (the occurrence-list kernel then writes every row).
+    uint8_t* row_live;
+    const uint32_t* live_off;
 };
+constexpr uint32_t kRowLiveStride = 128;  // a scan has at most 128 king blocks
 
 // The block-scan FT backward (ft_grad_scan_kernel): the forward's king-block
 // schedule, per-row hit masks and the flag that hands a step to the

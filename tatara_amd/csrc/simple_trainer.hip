@@ -67,6 +67,7 @@ class SimpleTrainer final : public TrainerBase {
     // block-scan FT backward (factorized feature sets)
     bool use_scan = false;
     uint32_t* scan_multi = nullptr;
+    uint8_t* row_live = nullptr;  // rows with an occurrence (FtGradArgs), or null
     uint32_t *scan_stage_rows = nullptr, *scan_stage_masks = nullptr;  // the block scan's stage tables
     // activations
     float *ft_stm = nullptr, *ft_nstm = nullptr, *combined = nullptr, *dft = nullptr;
@@ -177,6 +178,9 @@ class SimpleTrainer final : public TrainerBase {
                                            ft_scan_max_stages(B, n_king_bins) * ft_scan_mask_words(pi) * 16, false)) ||
                          (st = arena.alloc(&radix_hist, 256ull * binsort_tiles((uint32_t)n_items), false)) ||
                          (st = arena.alloc(&radix_count, 256))))
+            return st;
+        if (use_scan && n_king_bins <= kRowLiveStride && !keep &&
+            (st = arena.alloc(&row_live, (uint64_t)pi * kRowLiveStride)))
             return st;
         if ((st = arena.alloc(&ft_stm, B * ft_out, false)) || (st = arena.alloc(&ft_nstm, B * ft_out, false)) ||
             (st = arena.alloc(&combined, B * K, false)) || (st = arena.alloc(&dft, 2 * B * dft_chunks() * kDftChunk, false)) ||
@@ -481,6 +485,8 @@ class SimpleTrainer final : public TrainerBase {
         fb.v = ft.v;
         fb.slow = ft.slow;
         fb.grad = ft.grad;
+        fb.row_live = row_live;
+        fb.live_off = scan_multi;
         fb.ft_out = ft_out;
         fb.rows = ft_in;
         fb.apply_update = 1;

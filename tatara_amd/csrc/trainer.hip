@@ -112,6 +112,7 @@ class LayerStackTrainer final : public TrainerBase {
     // block-scan FT backward (f32 dft, factorized feature sets)
     bool use_scan = false;
     uint32_t* scan_multi = nullptr;
+    uint8_t* row_live = nullptr;  // rows with an occurrence (FtGradArgs), or null
     uint32_t *scan_stage_rows = nullptr, *scan_stage_masks = nullptr;  // the block scan's stage tables
     // activations
     float *ft_stm = nullptr, *ft_nstm = nullptr, *combined = nullptr, *dft = nullptr;
@@ -249,6 +250,9 @@ class LayerStackTrainer final : public TrainerBase {
                                            ft_scan_max_stages(B, n_king_bins) * ft_scan_mask_words(pi) * 16, false)) ||
                          (st = arena.alloc(&radix_hist, 256ull * binsort_tiles((uint32_t)n_items), false)) ||
                          (st = arena.alloc(&radix_count, 256))))
+            return st;
+        if (use_scan && n_king_bins <= kRowLiveStride && !keep && !h_out &&
+            (st = arena.alloc(&row_live, (uint64_t)pi * kRowLiveStride)))
             return st;
         const uint64_t dft_n = 2 * B * dft_chunks() * kDftChunk;
         if (h_out) {
@@ -629,6 +633,8 @@ class LayerStackTrainer final : public TrainerBase {
         fb.mirror16 = (h_fwd && !factorized) ? fwd16 : nullptr;
         fb.slow = ft.slow;
         fb.grad = ft.grad;
+        fb.row_live = row_live;
+        fb.live_off = scan_multi;
         fb.ft_out = ft_out;
         fb.rows = ft_in;
         fb.apply_update = 1;

@@ -73,3 +73,34 @@ def test_dense_gradients_beside_the_table_gradient(gpu, arch):
             out.append([np.array(losses)] + [t.get(n, k) for n in groups for k in ("w", "m", "v")])
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("arch", ["simple", "layerstack"])
+def test_rows_without_an_occurrence(gpu, arch):
+    """Gradients of absent rows unwritten against a trainer that keeps every
+    gradient: equal bits over batches whose rows come and go (what an earlier
+    step left in the gradients is not used), one position, and a batch with a
+    feature of another king block (every gradient comes from the other kernel)."""
+    out = []
+    for keep in (False, True):
+        if arch == "simple":
+            _, cfg = gs.make(ft_out=256, l1=32, l2=32, optimizer="adamw", b=64)
+            cfg.keep_grads = keep
+            t, groups = SimpleTrainer(cfg), SIMPLE_GROUPS
+        else:
+            sh, cfg = gt.make(ft_out=512, l1=16, l2=32, b=64, factorize=True)
+            cfg.keep_grads = keep
+            t, groups = LayerStackTrainer(cfg), GROUPS
+        with t:
+            for b, seed, stray in ((64, 1, False), (16, 2, False), (32, 3, True), (48, 4, False)):
+                if arch == "simple":
+                    args = (gs.batch_for(seed, b),)
+                else:
+                    args = gt.batch_for(seed, b, sh.nb)
+                if stray:
+                    idx = args[0].stm_indices.reshape(b, -1)
+                    idx[5, 0] = (int(idx[5, 0]) + cfg.piece_inputs) % cfg.ft_in
+                t.train_step(*args, 1e-2, 0.25, Sigmoid())
+            out.append([t.get(n, k) for n in groups for k in ("w", "m", "v")])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
