@@ -484,9 +484,12 @@ class LayerStackTrainer final : public TrainerBase {
         }
         // king-block schedule for the gather
         const int32_t* sched = nullptr;
-        if (factorized) {
+        const bool ordered = fb_off || gather_ordered(b, max_active, (h_fwd ? 2ull : 4ull) * ft_out, train != 0);
+        if (factorized && (ordered || (train && use_scan))) {
+            const hipStream_t ks = ordered ? stream : side;
+            if (!ordered && (st = fork_side())) return st;
             if ((st = launch_king_block_keys(p.stm, p.nstm, p.nnz, sched_keys, b, max_active, ft_in, pi,
-                                             n_king_bins, stream, fb_off, fb_bad)))
+                                             n_king_bins, ks, fb_off, fb_bad)))
                 return st;
             BinSortArgs bs{};
             bs.keys = sched_keys;
@@ -498,15 +501,15 @@ class LayerStackTrainer final : public TrainerBase {
             bs.bin_start = sched_start;
             bs.bin_count = sched_count;
             bs.out = schedule;
-            if ((st = launch_binsort(bs, stream))) return st;
-            sched = schedule;
+            if ((st = launch_binsort(bs, ks))) return st;
+            if (ordered) sched = schedule;
             if (train && use_scan) {
                 // hit masks of the block-scan backward, beside the forward,
                 // then the occurrence sort, which runs only when a row has
                 // features of two king blocks or one feature twice (the
                 // mask pass sets scan_multi); no host wait.  A batch passed
                 // as king-blocked (on_device = 2) queues no sort.
-                if ((st = fork_side())) return st;
+                if (ordered && (st = fork_side())) return st;
                 if ((st = launch_ft_scan_tables(block_scan(p), side))) return st;
                 if ((st = batch_king_blocked ? note_king_blocked_tables() : sort_occurrences(p, side, true)))
                     return st;

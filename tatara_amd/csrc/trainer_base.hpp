@@ -51,6 +51,20 @@ struct BatchPtrs {
     uint32_t b = 0;
 };
 
+// Whether the row-gather forward reads its rows by king block.  The order costs a
+// sort ahead of the forward (12 to 20 us) and pays by rows found in L2; as long as
+// the bytes that the batch gathers stay below the last-level cache's size it does
+// not.  Microseconds a call, ordered / by position:
+//   validate  Simple 256 b 256 102/68, 1024 106/76, 4096 (319 MB) 122/110, 8192
+//             138/150; LS 768 b 256 125/112, 1008 (248 MB) 136/132, 4096 180/228;
+//             LS 1536 b 1008 (495 MB) 168/170, 4096 286/365
+//   a step (the gradient's tables need the sort too, then beside the forward)
+//             Simple 256 b 256 310/302, 1024 (80 MB) 327/322, 4096 368/383; LS 768
+//             b 256 518/503, 1008 566/548, 4096 675/689; LS 1536 b 1008 1017/1005
+inline bool gather_ordered(uint64_t batch, uint32_t max_active, uint64_t row_bytes, bool train) {
+    return 2 * batch * max_active * row_bytes > (train ? 128ull << 20 : 256ull << 20);
+}
+
 class TrainerBase {
    public:
     static constexpr int kPhases = 7;  // prep, ft_forward, dense_forward, dense_backward,

@@ -69,3 +69,34 @@ def test_simple_forward_on_both_sides(gpu, kb, pi, ma, ft_out, line):
             for name, key, n in (("ft_stm_out", "ft_stm", 1), ("ft_nstm_out", "ft_nstm", 1), ("combined", "combined", 2)):
                 assert np.array_equal(t.activation(name, n * b * ft_out), a[key]), (b, name)
             assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
+
+
+# The row gather takes the positions by king block from 256 MB of gathered rows
+# (validation) or 128 MB (a step) on, and in the batch's order below.
+@pytest.mark.parametrize("arch,ft_out", [("simple", 512), ("layerstack", 1280), ("mixed", 1280)])
+@pytest.mark.parametrize("train", [False, True])
+def test_row_gather_in_either_order(gpu, arch, ft_out, train):
+    kb, pi, ma = 100, 128, 40
+    spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
+    lo = (128 if train else 256) * 2 ** 20 // (2 * ma * ft_out * (2 if arch == "mixed" else 4)) // 16 * 16
+    batch, bucket = a_batch(lo + 16, spec, lo)
+    first = Batch(batch.stm_indices[:lo], batch.nstm_indices[:lo], batch.nnz[:lo], batch.score[:lo], batch.wdl[:lo])
+    out = []
+    for b, args in ((lo, (first, bucket[:lo])), (lo + 16, (batch, bucket))):
+        shape = dict(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, max_batch=lo + 16)
+        if arch == "simple":
+            cfg = SimpleConfig(l1_out=32, l2_out=32, **shape)
+            cls, args = SimpleTrainer, args[:1]
+        else:
+            cfg = LayerStackConfig(num_buckets=8, **shape)
+            cfg, cls = cfg.all_optim() if arch == "mixed" else cfg, LayerStackTrainer
+        with cls(cfg) as t:
+            if train:
+                t.train_step(*args, 1e-3, 0.0, Wrm())
+            else:
+                t.validate_step(*args, 0.0, Wrm())
+            wide = ft_out * (2 if arch == "simple" else 1)
+            out.append([t.activation(n, b * w)[:lo * w] for n, w in
+                        (("ft_stm_out", ft_out), ("ft_nstm_out", ft_out), ("combined", wide))])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
