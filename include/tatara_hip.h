@@ -163,9 +163,9 @@ TATARA_API int32_t tatara_op_ft_weight_grad(const float* dft, const int32_t* stm
  * walked once in (perspective, position) order and added to the features of
  * the block that occur in them, so every cell is the same sequential sum as
  * sparse_ft_backward.rs:247-267 (stm then nstm).  A batch with a row whose
- * features lie in two king blocks (piece_inputs rows each) is computed from
- * occurrence lists instead; *used_block_scan (optional) reports which path
- * ran.  Overwrites grad rows [0, cols).  Synchronises. */
+ * features lie in two king blocks (piece_inputs rows each), and any batch of
+ * a table of more than 128 king blocks, is computed from occurrence lists
+ * instead; *used_block_scan (optional) reports which path ran.  Overwrites grad rows [0, cols).  Synchronises. */
 TATARA_API int32_t tatara_op_ft_weight_grad_blocked(const float* dft, const int32_t* stm_idx,
                                          const int32_t* nstm_idx, const int32_t* nnz, float* grad,
                                          uint32_t batch, uint32_t ft_out, uint32_t cols,

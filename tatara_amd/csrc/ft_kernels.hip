@@ -2252,6 +2252,10 @@ uint32_t ft_scan_mask_words(uint32_t piece_inputs) {
     return piece_inputs > 0 && g.words <= (uint32_t)kScanMaxWords ? g.words : 0u;
 }
 
+bool ft_scan_ok(uint32_t cols, uint32_t piece_inputs) {
+    return ft_scan_mask_words(piece_inputs) > 0 && ceil_div(cols, piece_inputs) <= kScanMaxBlocks;
+}
+
 uint64_t ft_scan_max_stages(uint32_t batch, uint32_t n_blocks) {
     return (2ull * batch + kScanStage - 1) / kScanStage + n_blocks;
 }
@@ -2259,7 +2263,8 @@ uint64_t ft_scan_max_stages(uint32_t batch, uint32_t n_blocks) {
 int32_t launch_ft_scan_tables(const FtBlockScan& s, hipStream_t stream) {
     TATARA_REQUIRE(ft_scan_mask_words(s.piece_inputs) > 0, "block scan: piece_inputs out of range");
     TATARA_REQUIRE(s.max_active <= (uint32_t)kMaxActive, "max_active must be <= 64");
-    TATARA_REQUIRE(s.n_blocks >= 1 && s.n_blocks <= 128, "block scan: 1 to 128 king blocks");
+    TATARA_REQUIRE(s.n_blocks >= 1 && s.n_blocks <= kScanMaxBlocks && s.n_blocks == ceil_div(s.cols, s.piece_inputs),
+                   "block scan: a bin for each of 1 to 128 king blocks");
     TATARA_REQUIRE(s.stage_rows && s.stage_masks && s.multi, "block scan: stage tables and flag");
     int32_t st = launch_fill_i32(reinterpret_cast<int32_t*>(s.multi), 1, 0, stream);
     if (st) return st;
@@ -2290,7 +2295,8 @@ int32_t launch_ft_grad_scan(const FtGradArgs& a, const FtBlockScan& s, hipStream
     TATARA_REQUIRE(a.ft_out % 4 == 0 && a.rows == s.cols, "block scan: shapes");
     TATARA_REQUIRE(moment_scales_ok(a), "f16 moment scales must be powers of two");
     const ScanGeom geom = scan_geom(s.piece_inputs);
-    TATARA_REQUIRE(s.n_blocks <= 128, "block scan: at most 128 king blocks");
+    TATARA_REQUIRE(s.n_blocks <= kScanMaxBlocks && s.n_blocks == ceil_div(s.cols, s.piece_inputs),
+                   "block scan: a bin for each of at most 128 king blocks");
     const uint64_t pairs = (uint64_t)ceil_div(a.ft_out, kDftChunk) * s.n_blocks;
     const uint64_t grid = (pairs + kNumXcd - 1) / kNumXcd * kNumXcd * geom.n_groups;
     if (grid > 0) {
@@ -2333,7 +2339,8 @@ int32_t launch_ft_grad_mfma(const FtGradArgs& a, const FtBlockScan& s, hipStream
     TATARA_REQUIRE(strided || dft_chunk_major(a, s.batch), "mfma backward: chunk-major dft, or row-major in whole chunks");
     TATARA_REQUIRE(a.ft_out % 4 == 0 && a.rows == s.cols, "mfma backward: shapes");
     TATARA_REQUIRE(moment_scales_ok(a), "f16 moment scales must be powers of two");
-    TATARA_REQUIRE(s.n_blocks <= 128, "mfma backward: at most 128 king blocks");
+    TATARA_REQUIRE(s.n_blocks <= kScanMaxBlocks && s.n_blocks == ceil_div(s.cols, s.piece_inputs),
+                   "mfma backward: a bin for each of at most 128 king blocks");
     TATARA_REQUIRE(!s.dealt, "mfma backward: stage tables with contiguous waves");
     const ScanGeom geom = scan_geom(s.piece_inputs);
     TATARA_REQUIRE(geom.group_size <= 128, "mfma backward: at most 128 features per group");
@@ -2360,6 +2367,8 @@ int32_t launch_ft_virtual_fold(const FtGradArgs& a, uint32_t piece_inputs, float
     TATARA_REQUIRE(piece_inputs > 0 && a.rows % piece_inputs == 0,
                    "virtual fold: rows must be a multiple of piece_inputs");
     TATARA_REQUIRE(a.grad, "virtual fold needs the real-row gradients");
+    TATARA_REQUIRE(!a.row_live || (a.live_off && a.rows / piece_inputs <= kRowLiveStride),
+                   "virtual fold: a flag for each of at most 128 king blocks");
     TATARA_REQUIRE(moment_scales_ok(a), "f16 moment scales must be powers of two");
     TATARA_REQUIRE(!(comb && comb16), "virtual fold writes one forward table");
     TATARA_REQUIRE(table_layout_ok(layout, comb16 != nullptr, a.ft_out), "virtual fold: table layout");

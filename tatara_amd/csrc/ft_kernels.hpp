@@ -116,7 +116,8 @@ struct FtGradArgs {
     uint8_t* row_live;
     const uint32_t* live_off;
 };
-constexpr uint32_t kRowLiveStride = 128;  // a scan has at most 128 king blocks
+constexpr uint32_t kScanMaxBlocks = 128;  // king blocks of a block scan
+constexpr uint32_t kRowLiveStride = kScanMaxBlocks;
 
 // The block-scan FT backward (ft_grad_scan_kernel): the forward's king-block
 // schedule, per-row hit masks and the flag that hands a step to the
@@ -159,6 +160,10 @@ int32_t launch_occurrence_sort(const OccurrenceSortArgs& a, hipStream_t stream);
 int32_t launch_ft_grad_update(const FtGradArgs& a, hipStream_t stream);
 // Mask words per schedule entry (0 when the block scan cannot serve piece_inputs).
 uint32_t ft_scan_mask_words(uint32_t piece_inputs);
+// Whether the block scan serves a table of `cols` rows: mask words, and a bin for
+// every king block (the schedule puts the rows of all blocks past its last bin
+// into that bin, so a scan over fewer bins than blocks would miss rows).
+bool ft_scan_ok(uint32_t cols, uint32_t piece_inputs);
 // Stages of 32 rows the block scan's tables hold at most for a batch.
 uint64_t ft_scan_max_stages(uint32_t batch, uint32_t n_blocks);
 // The block scan's stage tables and the multi flag of a batch (after its

@@ -379,8 +379,9 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
     TATARA_REQUIRE(max_active <= 64, "max_active must be <= 64");
     TATARA_REQUIRE(ft_scan_mask_words(piece_inputs) > 0, "piece_inputs out of range for the block scan");
     int32_t st;
-    uint32_t n_blocks = ceil_div(cols, piece_inputs);
-    if (n_blocks > 128) n_blocks = 128;
+    // a table of more king blocks than the schedule has bins: occurrence lists
+    const bool scan = ft_scan_ok(cols, piece_inputs);
+    const uint32_t n_blocks = scan ? ceil_div(cols, piece_inputs) : 0;
     const uint64_t two_b = 2ull * batch;
     // a row-major dft of whole column chunks, four values aligned, is read where
     // it lies; else its rows are laid out in chunks first (a value a lane where
@@ -392,27 +393,13 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
     const uint64_t chunk_bytes = in_place ? 0 : elem * ceil_div(ft_out, kDftChunk) * two_b * kDftChunk;
     // king-block schedule, as the trainer builds it for the forward
     DevCarve ws;
-    const uint64_t stages = ft_scan_max_stages(batch, n_blocks);
+    const uint64_t stages = scan ? ft_scan_max_stages(batch, n_blocks) : 0;
     const size_t keys = ws.add(two_b), sched = ws.add(4 * two_b),
                  hist = ws.add(4ull * 2 * n_blocks * binsort_tiles((uint32_t)two_b)),
                  start = ws.add(4ull * (2 * n_blocks + 1)), count = ws.add(4ull * 2 * n_blocks),
                  multi = ws.add(4), srows = ws.add(4ull * stages * 32),
                  smasks = ws.add(4ull * stages * ft_scan_mask_words(piece_inputs) * 16), cm = ws.add(chunk_bytes);
     if ((st = ws.alloc())) return st;
-    if ((st = launch_king_block_keys(stm_idx, nstm_idx, nnz, ws.take<uint8_t>(keys), batch, max_active, cols,
-                                     piece_inputs, n_blocks, 0)))
-        return st;
-    BinSortArgs bs{};
-    bs.keys = ws.take<uint8_t>(keys);
-    bs.n_items = (uint32_t)two_b;
-    bs.n_bins = 2 * n_blocks;
-    bs.align = 1;
-    bs.value_mod = batch;
-    bs.hist = ws.take<uint32_t>(hist);
-    bs.bin_start = ws.take<uint32_t>(start);
-    bs.bin_count = ws.take<uint32_t>(count);
-    bs.out = ws.take<int32_t>(sched);
-    if ((st = launch_binsort(bs, 0))) return st;
     if (!in_place && two_b * ft_out > 0) {
         const uint32_t per = aligned ? 4 : 1, row_v = ft_out / per, chunk_v = kDftChunk / per;
         const uint32_t blocks = ceil_div(two_b * row_v, 256);
@@ -426,22 +413,6 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
             aligned ? copy(static_cast<float4*>(nullptr)) : copy(static_cast<float*>(nullptr));
         TATARA_LAUNCHED("to_chunk_major");
     }
-    FtBlockScan sc{};
-    sc.idx_stm = stm_idx;
-    sc.idx_nstm = nstm_idx;
-    sc.nnz = nnz;
-    sc.schedule = ws.take<int32_t>(sched);
-    sc.sched_start = ws.take<uint32_t>(start);
-    sc.multi = ws.take<uint32_t>(multi);
-    sc.stage_rows = ws.take<uint32_t>(srows);
-    sc.stage_masks = ws.take<uint32_t>(smasks);
-    sc.batch = batch;
-    sc.max_active = max_active;
-    sc.cols = cols;
-    sc.piece_inputs = piece_inputs;
-    sc.n_blocks = n_blocks;
-    sc.dealt = mfma ? 0u : 1u;
-    if ((st = launch_ft_scan_tables(sc, 0))) return st;
     FtGradArgs g{};
     if (dft16) {
         g.dft16 = in_place ? dft16 : ws.take<uint16_t>(cm);
@@ -455,11 +426,43 @@ static int32_t ft_weight_grad_blocked(const float* dft, const uint16_t* dft16, f
     g.ft_out = ft_out;
     g.rows = cols;
     g.apply_update = 0;
-    // (does nothing when the tables found a row the scan cannot take)
-    if ((st = mfma ? launch_ft_grad_mfma(g, sc, 0, false) : launch_ft_grad_scan(g, sc, 0, false))) return st;
-    uint32_t m = 0;
-    TATARA_HIP(hipMemcpy(&m, sc.multi, 4, hipMemcpyDeviceToHost), "ft_weight_grad_blocked");
-    if (m) {  // a row with features of two blocks, or one twice: occurrence lists
+    uint32_t m = 1;
+    if (scan) {
+        if ((st = launch_king_block_keys(stm_idx, nstm_idx, nnz, ws.take<uint8_t>(keys), batch, max_active, cols,
+                                         piece_inputs, n_blocks, 0)))
+            return st;
+        BinSortArgs bs{};
+        bs.keys = ws.take<uint8_t>(keys);
+        bs.n_items = (uint32_t)two_b;
+        bs.n_bins = 2 * n_blocks;
+        bs.align = 1;
+        bs.value_mod = batch;
+        bs.hist = ws.take<uint32_t>(hist);
+        bs.bin_start = ws.take<uint32_t>(start);
+        bs.bin_count = ws.take<uint32_t>(count);
+        bs.out = ws.take<int32_t>(sched);
+        if ((st = launch_binsort(bs, 0))) return st;
+        FtBlockScan sc{};
+        sc.idx_stm = stm_idx;
+        sc.idx_nstm = nstm_idx;
+        sc.nnz = nnz;
+        sc.schedule = ws.take<int32_t>(sched);
+        sc.sched_start = ws.take<uint32_t>(start);
+        sc.multi = ws.take<uint32_t>(multi);
+        sc.stage_rows = ws.take<uint32_t>(srows);
+        sc.stage_masks = ws.take<uint32_t>(smasks);
+        sc.batch = batch;
+        sc.max_active = max_active;
+        sc.cols = cols;
+        sc.piece_inputs = piece_inputs;
+        sc.n_blocks = n_blocks;
+        sc.dealt = mfma ? 0u : 1u;
+        if ((st = launch_ft_scan_tables(sc, 0))) return st;
+        // (does nothing when the tables found a row the scan cannot take)
+        if ((st = mfma ? launch_ft_grad_mfma(g, sc, 0, false) : launch_ft_grad_scan(g, sc, 0, false))) return st;
+        TATARA_HIP(hipMemcpy(&m, sc.multi, 4, hipMemcpyDeviceToHost), "ft_weight_grad_blocked");
+    }
+    if (m) {  // a row with features of two blocks, or one twice, or too many blocks: occurrence lists
         OccurrenceLists occ;
         if ((st = occ.sort(stm_idx, nstm_idx, nnz, batch, max_active, cols))) return st;
         g.occ_vals = occ.vals;

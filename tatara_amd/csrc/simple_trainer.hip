@@ -171,7 +171,7 @@ class SimpleTrainer final : public TrainerBase {
             (st = arena.alloc(&occ_off, 2ull * ft_in + 2)) ||
             (st = arena.alloc((uint8_t**)&occ_tmp, occ_tmp_bytes, false)))
             return st;
-        use_scan = factorized && ft_out >= kDftChunk && ft_scan_mask_words(pi) > 0;
+        use_scan = factorized && ft_out >= kDftChunk && ft_scan_ok(ft_in, pi);
         if (use_scan && ((st = arena.alloc(&scan_multi, 1)) ||
                          (st = arena.alloc(&scan_stage_rows, ft_scan_max_stages(B, n_king_bins) * 32, false)) ||
                          (st = arena.alloc(&scan_stage_masks,
@@ -179,7 +179,7 @@ class SimpleTrainer final : public TrainerBase {
                          (st = arena.alloc(&radix_hist, 256ull * binsort_tiles((uint32_t)n_items), false)) ||
                          (st = arena.alloc(&radix_count, 256))))
             return st;
-        if (use_scan && n_king_bins <= kRowLiveStride && !keep &&
+        if (use_scan && !keep &&
             (st = arena.alloc(&row_live, (uint64_t)pi * kRowLiveStride)))
             return st;
         if ((st = arena.alloc(&ft_stm, B * ft_out, false)) || (st = arena.alloc(&ft_nstm, B * ft_out, false)) ||

@@ -243,7 +243,7 @@ class LayerStackTrainer final : public TrainerBase {
             (st = arena.alloc((uint8_t**)&occ_tmp, occ_tmp_bytes, false)))
             return st;
         // the block scan (f32 dft) or its matrix-core form (f16 dft)
-        use_scan = factorized && ft_out >= 2 * kDftChunk && ft_scan_mask_words(pi) > 0;
+        use_scan = factorized && ft_out >= 2 * kDftChunk && ft_scan_ok(ft_in, pi);
         if (use_scan && ((st = arena.alloc(&scan_multi, 1)) ||
                          (st = arena.alloc(&scan_stage_rows, ft_scan_max_stages(B, n_king_bins) * 32, false)) ||
                          (st = arena.alloc(&scan_stage_masks,
@@ -251,7 +251,7 @@ class LayerStackTrainer final : public TrainerBase {
                          (st = arena.alloc(&radix_hist, 256ull * binsort_tiles((uint32_t)n_items), false)) ||
                          (st = arena.alloc(&radix_count, 256))))
             return st;
-        if (use_scan && n_king_bins <= kRowLiveStride && !keep && !h_out &&
+        if (use_scan && !keep && !h_out &&
             (st = arena.alloc(&row_live, (uint64_t)pi * kRowLiveStride)))
             return st;
         const uint64_t dft_n = 2 * B * dft_chunks() * kDftChunk;
