@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kPsvWaves * 64) void psv_to_batch_kernel(PsvArgs a)
     constexpr int R = kPsvRecords;
     __shared__ uint32_t s_rec[R * 10];
     __shared__ uint16_t s_key[R * kKeyStride];  // (kind * 2 + colour) << 7 | square (hand: count - 1)
-    // flags (1 kings valid, 2 square maps of both sides << 2), board pieces, pieces; the
+    // flags (1 kings valid, 2 a hand past its range, 2 square maps of both sides << 2), board pieces, pieces; the
     // sides' feature bases; their two king features; the kings' progress rows
     __shared__ int32_t s_meta[R][9];
     __shared__ uint8_t s_map[4][96];  // square by (white's view, mirrored file)
@@ -213,7 +213,12 @@ __global__ __launch_bounds__(kPsvWaves * 64) void psv_to_batch_kernel(PsvArgs a)
             s_meta[t][6] = base_n + enemy + mirror_sq(persp_sq(ks, nstm), mir_n);
             s_meta[t][7] = (int)king0 * kFeOldEnd;
             s_meta[t][8] = (80 - (int)king1) * kFeOldEnd;
-            s_meta[t][0] = (int)(1u | (stm * 2 + mir_s) << 2 | (nstm * 2 + mir_n) << 4 | n_board << 8 | n_piece << 16);
+            // More pieces in a hand than a set has (rooks: three or more) reach past
+            // the hands' range, where the reference's pack_bonapiece mirrors: a
+            // hand of more than 90 - (its base as the enemy's), a byte each.
+            constexpr uint64_t kPast = 0x7d776f655b5139ull;  // 127 - (70, 46, 36, 26, 16, 8, 2), pawns lowest
+            const bool past = a.mirror && (((hand0 + kPast) | (hand1 + kPast)) & 0x80808080808080ull);
+            s_meta[t][0] = (int)(1u | (past ? 2u : 0u) | (stm * 2 + mir_s) << 2 | (nstm * 2 + mir_n) << 4 | n_board << 8 | n_piece << 16);
         } else {
             s_meta[t][0] = 0;
         }
@@ -276,6 +281,12 @@ __global__ __launch_bounds__(kPsvWaves * 64) void psv_to_batch_kernel(PsvArgs a)
         // (a hand's count goes through the identity map)
         int f_s = base_s + (friend_s ? base_f : base_e) + s_map[board ? map_s : 0u][sq];
         int f_n = base_n + (friend_s ? base_e : base_f) + s_map[board ? map_n : 0u][sq];
+        if (meta & 2u) {  // a hand past the hands' range: mirrored as a board piece's square
+            const int over_f = base_f + (int)sq - kFeHandEnd, over_e = base_e + (int)sq - kFeHandEnd;
+            const int over_s = friend_s ? over_f : over_e, over_n = friend_s ? over_e : over_f;
+            if (piece && !board && over_s >= 0) f_s = base_s + kFeHandEnd + s_map[map_s & 1u][over_s];
+            if (piece && !board && over_n >= 0) f_n = base_n + kFeHandEnd + s_map[map_n & 1u][over_n];
+        }
         if (!piece) {
             const uint32_t e = lane - n_piece;  // past the pieces
             const bool king = e < n_king;

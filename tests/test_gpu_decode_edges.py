@@ -30,6 +30,33 @@ def crafted():
     return np.stack(recs)
 
 
+def full_hands():
+    """An empty board and one hand of every count of one piece, up to a record's
+    room.  From three rooks on, the hand's feature is no longer below the board's
+    first (90), where the reference mirrors it like a board piece's."""
+    codes = {2: [1, 0, 0], 4: [1, 1, 0], 5: [1, 1, 1, 0], 6: [1, 1, 1, 1, 0], 7: [1, 1, 1, 1, 1]}  # first bit lowest
+    recs = []
+    for piece, code in codes.items():
+        entry = code + ([] if piece == 5 else [0])  # not in the piece box (gold has no such bit)
+        for owner in (0, 1):
+            for count in range(1, 162 // (len(entry) + 1) + 1):
+                kings = (count * 7 % 81, (count * 31 + 40) % 81)
+                head = (count & 1) | kings[0] << 1 | kings[1] << 8
+                bits = [(head >> i) & 1 for i in range(15)] + [0] * (81 - len(set(kings)))
+                bits += (entry + [owner]) * count
+                bits += [0, 1, 0] * 60  # pawns in the piece box
+                rec = np.zeros(40, np.uint8)
+                rec[:32] = np.packbits(np.array(bits[:256], np.uint8), bitorder="little")
+                recs.append(rec)
+    return np.stack(recs)
+
+
+@pytest.mark.parametrize("fs", FS)
+def test_hands_of_any_count(gpu, fs):
+    compare(full_hands(), fs, "none")
+    compare(full_hands(), fs, "progress", 9, np.random.default_rng(3).normal(0.0, 0.05, 81 * 1548))
+
+
 @pytest.mark.parametrize("fs", FS)
 def test_record_counts_and_full_records(gpu, fs):
     rng = np.random.default_rng(9)
