@@ -495,6 +495,7 @@ class SimpleTrainer final : public TrainerBase {
         fb.apply_update = 1;
         fb.opt = scalars(0, lr, step_count);
         if (!profiling && ((st = fork_side()) || (st = finalize_dense()))) return st;
+        if ((st = join_lists())) return st;
         if ((st = ft_gradient(p, fb))) return st;
         if ((st = prof_mark(5))) return st;
         if (factorized && (st = launch_ft_virtual_fold(fb, pi, comb, nullptr, stream, table_layout()))) return st;

@@ -643,6 +643,7 @@ class LayerStackTrainer final : public TrainerBase {
         fb.apply_update = 1;
         fb.opt = sf;
         if (!profiling && ((st = fork_side()) || (st = finalize_dense()))) return st;
+        if ((st = join_lists())) return st;
         if ((st = ft_gradient(p, fb))) return st;
         if ((st = prof_mark(5))) return st;
         if (factorized &&

@@ -34,6 +34,7 @@ TrainerBase::~TrainerBase() {
     if (side) (void)hipStreamSynchronize(side);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
+    if (ev_lists) (void)hipEventDestroy(ev_lists);
     if (pinned_loss) (void)hipHostFree(pinned_loss);
     if (kb_ev) (void)hipEventDestroy(kb_ev);
     if (kb_broken_host) (void)hipHostFree(kb_broken_host);
@@ -47,6 +48,7 @@ int32_t TrainerBase::init_runtime(int device) {
     TATARA_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking), "hipStreamCreate (side)");
     TATARA_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming), "hipEventCreate");
     TATARA_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming), "hipEventCreate");
+    TATARA_HIP(hipEventCreateWithFlags(&ev_lists, hipEventDisableTiming), "hipEventCreate");
     TATARA_HIP(hipEventCreateWithFlags(&loss_ev[0], hipEventDisableTiming), "hipEventCreate");
     TATARA_HIP(hipEventCreateWithFlags(&loss_ev[1], hipEventDisableTiming), "hipEventCreate");
     TATARA_HIP(hipHostMalloc((void**)&pinned_loss, 2 * sizeof(double), hipHostMallocDefault),
@@ -330,6 +332,18 @@ int32_t TrainerBase::fork_side() {
 int32_t TrainerBase::join_side() {
     TATARA_HIP(hipEventRecord(ev_join, side), "hipEventRecord (join)");
     TATARA_HIP(hipStreamWaitEvent(stream, ev_join, 0), "hipStreamWaitEvent (join)");
+    return kOk;
+}
+
+int32_t TrainerBase::fork_dense() {
+    if (profiling) return kOk;
+    TATARA_HIP(hipEventRecord(ev_lists, side), "hipEventRecord (lists)");
+    return fork_side();
+}
+
+int32_t TrainerBase::join_lists() {
+    if (profiling) return join_side();
+    TATARA_HIP(hipStreamWaitEvent(stream, ev_lists, 0), "hipStreamWaitEvent (lists)");
     return kOk;
 }
 

@@ -161,7 +161,7 @@ class TrainerBase {
     int32_t note_king_blocked_tables();
     // phase profiling: kPhases + 1 events per profiled step
     std::vector<hipEvent_t> prof_events;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_lists = nullptr;
 
     int32_t init_runtime(int device);
     int32_t alloc_inputs(uint64_t max_b, uint32_t max_active);
@@ -200,14 +200,15 @@ class TrainerBase {
     // batch 2048 458 -> 445, LayerStack 768, batch 16384 1163 -> 1130; at 1536,
     // batch 65536 both sides are bound by memory (4057 -> 4046).  While phases are
     // profiled they stay on `stream`, so that each phase's time is its own.
-    // fork_dense: stream has what was queued on side before it, side what was
-    // queued on stream.
+    // fork_dense: side has what was queued on stream; join_lists: stream has what
+    // was queued on side before fork_dense, the table gradient's tables or lists.
+    // The stream waits for them just ahead of that gradient: a narrow table's
+    // occurrence sort ends after the forward and runs on beside the input
+    // gradient (waiting for it in fork_dense: LayerStack 128, b 65536, 1030 ->
+    // 1086 us a step).
     hipStream_t dense_stream() const { return profiling ? stream : side; }
-    int32_t fork_dense() {
-        int32_t st;
-        if ((st = join_side())) return st;
-        return profiling ? kOk : fork_side();
-    }
+    int32_t fork_dense();
+    int32_t join_lists();
 };
 
 // The stream a trainer handle's steps run on (work enqueued there before a
