@@ -1989,14 +1989,29 @@ bool ft_forward_block_ok(int mode, bool f16_table, uint32_t ft_out, uint32_t pie
 //      39.7       346 / 351  596 / 671  1176 / 1341
 // (and at 39.7, Simple 256, the L1 forward after the staged form finds more of
 // `combined` in the cache: 102 against 131).
+// A network too narrow for the block scan (LayerStack below 512, Simple below 256)
+// sorts its occurrences on the side stream from the forward on, and the step's
+// table gradient waits for that sort: the row gather leaves it less of the chip,
+// so the line lies lower.  A whole step, staged / rows, in us:
+//   occurrences   f32 128      f32 256      f32 384      f16 128      f16 256      f16 384
+//       8.9       293 / 291    371 / 352    539 / 532    274 / 272    321 / 309    443 / 414
+//      17.9       361 / 366    484 / 463    687 / 679    336 / 359    409 / 402    557 / 537
+//      35.8       543 / 598    698 / 734    972 / 1060   509 / 578    575 / 637    775 / 814
+//      71.5       990 / 1081   1280 / 1292  1679 / 1858  886 / 1019   1003 / 1104  1307 / 1379
+//   occurrences   Simple 32    Simple 64    Simple 128   Simple 192
+//       5.0       250 / 234    263 / 250    314 / 285    384 / 336
+//       9.9       302 / 318    316 / 330    378 / 378    464 / 451
+//      14.9       367 / 407    383 / 423    445 / 474    548 / 550
+//      29.8       574 / 659    605 / 691    698 / 779    847 / 928
 bool ft_forward_block_pays(int mode, bool f16_table, uint32_t ft_out, uint32_t cols, uint32_t max_active,
                            uint32_t batch) {
     uint64_t line;  // occurrences per table row
     if (mode == kConcat) {
-        line = ft_out <= 256 ? 32 : 20;
+        line = ft_out <= 64 ? 8 : ft_out <= 128 ? 10 : ft_out < 256 ? 14 : ft_out == 256 ? 32 : 20;
+    } else if (f16_table) {
+        line = ft_out <= 128 ? 12 : ft_out == 512 ? 80 : 20;
     } else {
-        if (ft_out <= 256) return false;
-        line = f16_table ? (ft_out <= 512 ? 80 : 20) : (ft_out < 768 ? 20 : 16);
+        line = ft_out <= 128 ? 16 : ft_out < 768 ? 20 : 16;
     }
     return 2ull * batch * max_active >= line * cols;
 }

@@ -33,7 +33,9 @@ def a_batch(b, spec, seed):
 # (king blocks, pieces, slots, columns, occurrences per table row on the line)
 @pytest.mark.parametrize("mixed,kb,pi,ma,ft_out,line",
                          [(False, 10, 64, 40, 512, 20), (False, 10, 64, 44, 640, 20), (False, 10, 64, 38, 768, 16),
-                          (False, 2, 1791, 40, 384, 20), (True, 10, 64, 40, 640, 20), (True, 10, 64, 44, 512, 80)])
+                          (False, 2, 1791, 40, 384, 20), (True, 10, 64, 40, 640, 20), (True, 10, 64, 44, 512, 80),
+                          (False, 10, 64, 40, 128, 16), (False, 10, 64, 38, 256, 20), (True, 10, 64, 44, 128, 12),
+                          (True, 10, 64, 40, 256, 20)])
 def test_layerstack_forward_on_both_sides(gpu, mixed, kb, pi, ma, ft_out, line):
     spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
     sh = ols.LsShape(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, l1=16, l2=32, nb=8)
@@ -53,7 +55,8 @@ def test_layerstack_forward_on_both_sides(gpu, mixed, kb, pi, ma, ft_out, line):
             assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
 
 
-@pytest.mark.parametrize("kb,pi,ma,ft_out,line", [(10, 64, 44, 256, 32), (10, 64, 38, 512, 20), (2, 1791, 40, 128, 32)])
+@pytest.mark.parametrize("kb,pi,ma,ft_out,line", [(10, 64, 44, 256, 32), (10, 64, 38, 512, 20), (2, 1791, 40, 128, 32),
+                                                  (10, 64, 40, 32, 8), (2, 1791, 38, 128, 10), (10, 64, 44, 224, 14)])
 def test_simple_forward_on_both_sides(gpu, kb, pi, ma, ft_out, line):
     spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
     sh = osi.SimpleShape(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, l1=32, l2=32)
