@@ -66,6 +66,13 @@ TATARA_API int32_t tatara_memcpy_dtoh(void* dst, const void* src, uint64_t bytes
 TATARA_API int32_t tatara_memset(void* dst, int32_t byte, uint64_t bytes);
 /* Waits for all work on the device (CudaStream::synchronize). */
 TATARA_API int32_t tatara_synchronize(void);
+/* Frees the device memory that the calling thread keeps for the standalone ops:
+ * tatara_op_ft_forward_pairwise, the tatara_op_ft_weight_grad calls and
+ * tatara_op_quantise_ft keep their scratch between calls, at most 64 MB a thread,
+ * until the thread ends, calls one of them on another device or calls this.
+ * Another library's hipDeviceReset between two calls does no harm: the next one
+ * allocates anew. */
+TATARA_API int32_t tatara_release_scratch(void);
 
 /* Streams, events, asynchronous copies, pinned host memory and code-object
  * modules: the rest of the runtime surface (native_backend.rs:33-300,

@@ -210,6 +210,7 @@ SIGNATURES = {
     "tatara_memcpy_dtoh": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_uint64]),
     "tatara_memset": (C.c_int32, [C.c_void_p, C.c_int32, C.c_uint64]),
     "tatara_synchronize": (C.c_int32, []),
+    "tatara_release_scratch": (C.c_int32, []),
     "tatara_device_occupancy_attributes": (C.c_int32, [C.c_int32, c_i32p, c_i32p]),
     "tatara_device_compute_capability": (C.c_int32, [C.c_int32, c_i32p, c_i32p]),
     "tatara_stream_create": (C.c_int32, [C.c_int32, C.POINTER(C.c_void_p)]),

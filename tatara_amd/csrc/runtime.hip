@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "export.hpp"
 #include "ft_kernels.hpp"
+#include "kept_scratch.hpp"
 #include "psv_kernels.hpp"
 
 namespace tatara {
@@ -57,25 +58,6 @@ struct DevScratch {
     }
 };
 
-// The scratch memory a thread keeps between ops: at most kKeptBytes on one
-// device, freed when the thread ends or asks for it on another device.  An op
-// has synchronised before it returns, so the memory is idle between calls.
-// Allocating and freeing these buffers on each call cost the f32 gradient op at
-// ft_out 768, batch 16381 110 us of 358 (now 239), the f16 one at 1536, 16384 118
-// us of 440 (now 321).  64 MB hold an op's lists up to a batch of about 100,000.
-constexpr size_t kKeptBytes = 64ull << 20;
-struct KeptScratch {
-    void* p = nullptr;
-    size_t bytes = 0;
-    int device = -1;
-    bool lent = false;
-    ~KeptScratch() { drop(); }
-    void drop() {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        bytes = 0;
-    }
-};
 thread_local KeptScratch g_kept;
 
 // Several buffers in one allocation, 256-byte aligned; the thread's kept
@@ -86,7 +68,7 @@ struct DevCarve {
     size_t bytes = 0;
     bool borrowed = false;
     ~DevCarve() {
-        if (borrowed) g_kept.lent = false;
+        if (borrowed) g_kept.give_back();
     }
     // the buffer's offset; take(offset) after alloc()
     size_t add(size_t n) {
@@ -95,19 +77,11 @@ struct DevCarve {
         return at;
     }
     int32_t alloc() {
-        if (bytes <= kKeptBytes && !g_kept.lent) {
-            int device = 0;
-            TATARA_HIP(hipGetDevice(&device), "hipGetDevice scratch");
-            if (g_kept.device != device || g_kept.bytes < bytes) {
-                g_kept.drop();
-                void* p = nullptr;
-                TATARA_HIP(hipMalloc(&p, bytes), "hipMalloc scratch");
-                g_kept.p = p;
-                g_kept.bytes = bytes;
-                g_kept.device = device;
-            }
-            g_kept.lent = borrowed = true;
-            base = static_cast<uint8_t*>(g_kept.p);
+        void* p = nullptr;
+        TATARA_HIP(g_kept.lend(bytes, &p), "scratch");
+        if (p) {
+            borrowed = true;
+            base = static_cast<uint8_t*>(p);
             return kOk;
         }
         const int32_t st = own.alloc(bytes);
@@ -230,6 +204,11 @@ int32_t tatara_memset(void* dst, int32_t byte, uint64_t bytes) {
 
 int32_t tatara_synchronize(void) {
     TATARA_HIP(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    return kOk;
+}
+
+int32_t tatara_release_scratch(void) {
+    g_kept.release();
     return kOk;
 }
 
