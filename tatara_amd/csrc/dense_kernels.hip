@@ -833,8 +833,19 @@ __global__ __launch_bounds__(256) void ls_l1_wgrad_kernel(LsDenseArgs a) {
 // 8-byte) pieces.
 // With the sums as per-column FMAs (32 an element, plus the dl1 broadcasts)
 // the kernel was bound by vector issue in f16.  ft_out 1536, b 65536: f16 273
-// -> 193 us (0.8 GB, 4.2 TB/s), f32 324 -> 330 (1.6 GB, 4.9 TB/s: memory);
-// ft_out 512, l1 32, b 2048: 25 -> 18 us.  The weights wait in LDS (each lane
+// -> 193 us (0.8 GB, 4.2 TB/s); ft_out 512, l1 32, b 2048: 25 -> 18 us.  In f32
+// memory bounds it (1.6 GB), and the step reads the raw sums here for the last
+// time: with plain loads they took the last-level cache from the dft rows being
+// written, and the kernel was slower than the per-column form it replaces.  The
+// dense backward of a step, per-column form / plain loads / non-temporal ones, in us:
+//   b 65536  ft 1536 l1 16  419 / 426 / 402   768 l1 8  202 / 210 / 194
+//            640 l1 16      179 / 187 / 172   512 l1 16 150 / 161 / 154
+//   b 32768  1152 l1 8      153 / 159 / 149   1024 l1 32 190 / 201 / 195
+//            768 l1 8       113 / 114 / 109   512 l1 32 119 / 124 / 124
+//   b 16384  1536 l1 16     118 / 121 / 116   768 l1 8  73 / 72 / 73
+//            512 l1 16      76 / 61 / 60;  b 2048  512 l1 32  54 / 48 / 48
+// (a whole step is not slower in any of them; workgroups of four waves gave 395 at
+// 1536 but cost the step 5% at 512 l1 16, b 65536.)  The weights wait in LDS (each lane
 // reads back what it wrote, so nothing is synchronised): in registers they
 // cost a wave per SIMD.  The next tile's raw sums loaded ahead measured
 // slower (255 us f16): 32 more registers, one wave per SIMD less.
@@ -922,8 +933,13 @@ __global__ __launch_bounds__(128) void ls_l1_input_post_kernel(LsDenseArgs a, ui
 #pragma unroll
             for (int r = 0; r < 4; ++r) {  // row 0 (always valid) where the row is padding
                 const uint64_t base = (uint64_t)(rows[r] >= 0 ? rows[r] : 0) * ft_out + p;
-                xr[r] = raw[base / 4];
-                yr[r] = raw[(base + half) / 4];
+                if constexpr (H16) {
+                    xr[r] = raw[base / 4];
+                    yr[r] = raw[(base + half) / 4];
+                } else {
+                    xr[r] = __builtin_nontemporal_load(raw + base / 4);
+                    yr[r] = __builtin_nontemporal_load(raw + (base + half) / 4);
+                }
             }
             if (cur.bin != cur_bin) {
                 cur_bin = cur.bin;
