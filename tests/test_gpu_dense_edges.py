@@ -9,6 +9,7 @@ from oracle import layerstack as ols
 from oracle import simple as osi
 from tatara_amd.trainer import GROUPS, SIMPLE_GROUPS, LayerStackTrainer, Sigmoid, SimpleTrainer
 
+import test_gpu_mixed as gm
 import test_gpu_simple as gs
 import test_gpu_trainer as gt
 
@@ -53,6 +54,33 @@ def test_layerstack_edges(gpu, ft_out, l1, l2, b, factorize):
             gt.close(t.activation(name, b * ft_out), a[name], 1e-4, atol=1e-5 * top, what=name)
         for name in GROUPS:
             gt.close(t.get(name, "grad"), g[name], 1e-4, atol_frac=1e-5, what=f"grad {name}")
+
+
+# The input gradient's row blocks hold eight tiles from tiles * ft_out / 64 = 32768
+# on: 1366 and 1367 tiles of 16 rows end in a block of 6 and 7 (f32 writes a whole
+# ft_b partial and a shorter one there, f16 one).  The mixed form below that at
+# columns of one and three workgroups.
+@pytest.mark.parametrize("mixed,ft_out,l1,b", [(False, 1536, 8, 21712), (False, 1536, 16, 21728), (True, 1536, 8, 21712),
+                                               (True, 1536, 32, 21728), (True, 128, 32, 272), (True, 384, 8, 1040)])
+def test_input_gradient_row_blocks(gpu, mixed, ft_out, l1, b):
+    prec = ols.Precision.all_optim() if mixed else ols.FP32
+    sh, cfg = gt.make(ft_out=ft_out, l1=l1, l2=16, b=b, factorize=False)
+    cfg = cfg.all_optim() if mixed else cfg
+    batch, bucket = gt.batch_for(b, b, sh.nb)
+    st = gm.oracle_state(sh, prec)
+    bf, loss = b * ft_out, Sigmoid()
+    with LayerStackTrainer(cfg) as t:
+        t.train_step(batch, bucket, 8.75e-4, 0.25, loss)
+        _, a, g = ols.train_step(sh, st, gt.as_dict(batch, bucket), ols.OptConfig(), 8.75e-4, 0.25,
+                                 gt.loss_dict(loss), 1, prec)
+        for name in ("dft_stm", "dft_nstm"):
+            if mixed:
+                gt.close(t.activation(name, bf), a[name + "16"], 2e-3, atol=gm.SUB16, what=name)
+            else:
+                gt.close(t.activation(name, bf), a[name], 1e-4, atol=1e-5 * np.abs(a[name]).max(), what=name)
+        for name in GROUPS:
+            if name != "ft_w":
+                gt.close(t.get(name, "grad"), g[name], 1e-4, atol_frac=1e-5, what=f"grad {name}")
 
 
 @pytest.mark.parametrize("arch", ["simple", "layerstack", "unfactorized"])
