@@ -361,7 +361,8 @@ TATARA_API int32_t tatara_wdl_at(const TataraWdlSchedule* schedule, uint64_t bat
 typedef struct TataraTrainerConfig {
     int32_t arch;          /* TATARA_ARCH_* */
     int32_t device;
-    int32_t max_batch;     /* workspace capacity in positions (multiple of 16) */
+    int32_t max_batch;     /* workspace capacity in positions (multiple of 16); chooses the FT forward's
+                            * form too: a smaller batch takes the one that is fastest for a full batch */
     int32_t ft_in;         /* base FT input rows of the feature set */
     int32_t max_active;    /* active-feature slots per perspective (<= 64) */
     int32_t piece_inputs;  /* factorizer piece inputs; 0 = factorizer off */

@@ -57,7 +57,9 @@ struct FtForwardArgs {
 // ft_out, piece_inputs, max_active); otherwise the row gather runs.
 bool ft_forward_block_ok(int mode, bool f16_table, uint32_t ft_out, uint32_t piece_inputs, uint32_t max_active);
 // Whether it is also the faster form for batches of `batch` positions (the
-// line and the measurements on both sides of it: the definition).
+// line and the measurements on both sides of it: the definition).  A trainer asks
+// once, for its capacity, since the two forms read tables of different layouts: a
+// small batch on a large trainer stages the whole table too.
 bool ft_forward_block_pays(int mode, bool f16_table, uint32_t ft_out, uint32_t cols, uint32_t max_active,
                            uint32_t batch);
 // Slots per row of FtForwardArgs::slot_off (max_active rounded up to 40 or 48;

@@ -52,17 +52,31 @@ struct BatchPtrs {
 };
 
 // Whether the row-gather forward reads its rows by king block.  The order costs a
-// sort ahead of the forward (12 to 20 us) and pays by rows found in L2; as long as
-// the bytes that the batch gathers stay below the last-level cache's size it does
-// not.  Microseconds a call, ordered / by position:
-//   validate  Simple 256 b 256 102/68, 1024 106/76, 4096 (319 MB) 122/110, 8192
-//             138/150; LS 768 b 256 125/112, 1008 (248 MB) 136/132, 4096 180/228;
-//             LS 1536 b 1008 (495 MB) 168/170, 4096 286/365
-//   a step (the gradient's tables need the sort too, then beside the forward)
-//             Simple 256 b 256 310/302, 1024 (80 MB) 327/322, 4096 368/383; LS 768
-//             b 256 518/503, 1008 566/548, 4096 675/689; LS 1536 b 1008 1017/1005
+// sort ahead of the forward (12 to 20 us; in a step of a block-scan network the
+// tables need it too, then beside the forward) and pays by rows found in L2, once
+// what the batch gathers has outgrown the last-level cache (256 MB): a little
+// later in validation, where the wait for the sort weighs more, and in a step not
+// below 2048 positions, where the sort's launches are as long as the forward.
+// Microseconds, by king block / by position (MB gathered):
+//   validate  LS f32 512    134/123 (160)  143/144 (320)  160/189 (640)
+//             f32 768       142/132 (236)  154/165 (480);  f32 1536 142/131 (240)  158/162 (473)
+//             f16 512       136/126 (160)  137/141 (320);  f16 768  144/140 (240)  158/170 (480)
+//             f16 1536      153/143 (236)  167/178 (480);  f32 256  125/119 (160)  135/141 (320)
+//             Simple 256    116/88 (152)   122/107 (304)  140/149 (608)
+//             Simple 512    135/117 (304)  151/157 (608);  Simple 128 126/101 (304)
+//   a step    LS f32 512 b 2048 433/429 (320), 4096 479/499;  768 b 1008 564/550 (236),
+//             2048 606/598 (480), 4096 678/698;  1536 b 1008 1020/1009 (473), 2048
+//             1096/1103, 4096 1213/1271
+//             f16 512 b 2048 377/369 (160), 4096 396/398 (320), 8192 428/459;  768 b
+//             2048 508/494 (240), 4096 540/541 (480), 8192 597/628;  1536 b 2048
+//             900/897 (480), 4096 952/977
+//             f32 256 b 2048 269/270 (160), 4096 299/309 (320);  384 b 2048 371/373
+//             (240), 4096 428/447;  128 b 4096 231/226 (160), 8192 286/280 (320)
+//             Simple 256 b 2048 342/334 (152), 4096 368/373 (304);  512 b 2048 613/605
+//             (304), 4096 667/672;  128 b 4096 245/242 (152), 8192 288/295 (304)
 inline bool gather_ordered(uint64_t batch, uint32_t max_active, uint64_t row_bytes, bool train) {
-    return 2 * batch * max_active * row_bytes > (train ? 128ull << 20 : 256ull << 20);
+    const uint64_t gathered = 2 * batch * max_active * row_bytes;
+    return train ? batch > 2048 && gathered > 256ull << 20 : gathered > 320ull << 20;
 }
 
 class TrainerBase {

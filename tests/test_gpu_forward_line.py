@@ -74,14 +74,16 @@ def test_simple_forward_on_both_sides(gpu, kb, pi, ma, ft_out, line):
             assert np.allclose(net, a["net"], rtol=1e-5, atol=1e-6), b
 
 
-# The row gather takes the positions by king block from 256 MB of gathered rows
-# (validation) or 128 MB (a step) on, and in the batch's order below.
-@pytest.mark.parametrize("arch,ft_out", [("simple", 512), ("layerstack", 1280), ("mixed", 1280)])
+# The row gather takes the positions by king block above 320 MB of gathered rows
+# (validation), or 256 MB and 2048 positions (a step), and in the batch's order
+# below.
+@pytest.mark.parametrize("arch,ft_out", [("simple", 512), ("simple", 256), ("layerstack", 1280), ("mixed", 1280)])
 @pytest.mark.parametrize("train", [False, True])
 def test_row_gather_in_either_order(gpu, arch, ft_out, train):
     kb, pi, ma = 100, 128, 40
     spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
-    lo = (128 if train else 256) * 2 ** 20 // (2 * ma * ft_out * (2 if arch == "mixed" else 4)) // 16 * 16
+    lo = (256 if train else 320) * 2 ** 20 // (2 * ma * ft_out * (2 if arch == "mixed" else 4)) // 16 * 16
+    lo = max(lo, 2048) if train else lo
     batch, bucket = a_batch(lo + 16, spec, lo)
     first = Batch(batch.stm_indices[:lo], batch.nstm_indices[:lo], batch.nnz[:lo], batch.score[:lo], batch.wdl[:lo])
     out = []
@@ -101,5 +103,33 @@ def test_row_gather_in_either_order(gpu, arch, ft_out, train):
             wide = ft_out * (2 if arch == "simple" else 1)
             out.append([t.activation(n, b * w)[:lo * w] for n, w in
                         (("ft_stm_out", ft_out), ("ft_nstm_out", ft_out), ("combined", wide))])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+
+
+# A trainer chooses by its capacity whether it stages the whole table or gathers
+# rows: the same small batch on a capacity far above the line and on one below it.
+@pytest.mark.parametrize("arch,ft_out", [("simple", 256), ("layerstack", 512), ("layerstack", 128), ("mixed", 640)])
+@pytest.mark.parametrize("train", [False, True])
+def test_small_batch_on_a_large_capacity(gpu, arch, ft_out, train):
+    kb, pi, ma, b = 10, 64, 40, 48
+    spec = small_spec(king_buckets=kb, piece_inputs=pi, max_active=ma)
+    batch, bucket = a_batch(b, spec, 7)
+    out = []
+    for capacity in (b, 4096):
+        shape = dict(ft_in=kb * pi, max_active=ma, piece_inputs=pi, ft_out=ft_out, max_batch=capacity)
+        if arch == "simple":
+            cfg, cls, args = SimpleConfig(l1_out=32, l2_out=32, **shape), SimpleTrainer, (batch,)
+        else:
+            cfg, cls, args = LayerStackConfig(num_buckets=8, **shape), LayerStackTrainer, (batch, bucket)
+            cfg = cfg.all_optim() if arch == "mixed" else cfg
+        with cls(cfg) as t:
+            if train:
+                t.train_step(*args, 1e-3, 0.0, Wrm())
+                t.flush_pending_loss()
+            wide = ft_out * (2 if arch == "simple" else 1)
+            got = [np.float64(t.validate_step(*args, 0.0, Wrm())[1])]  # with the weights after the step
+            out.append(got + [t.activation(n, b * w) for n, w in
+                              (("ft_stm_out", ft_out), ("ft_nstm_out", ft_out), ("combined", wide))])
     for x, y in zip(*out):
         assert np.array_equal(x, y)
