@@ -1157,7 +1157,15 @@ uint32_t ls_max_chunks(uint32_t padded_b, uint32_t nb) {
 //   4096      102 / 72         63 / 46       80 / 65        43 / 39
 //   8192      123 / 99         75 / 60       90 / 79        48 / 45
 //   16384     131 / 147        80 / 81       99 / 114       50 / 58
-constexpr uint32_t kL1PairTiles = 640;
+// The sums of few columns are short, and the line lies lower there.  A whole
+// training step (and the phase):
+//   b        ft 128 l1 8         ft 128 l1 32        ft 256 l1 8         ft 256 l1 32
+//   3072      221 / 215 (32/29)   240 / 236 (42/38)   298 / 289 (37/29)   326 / 311 (53/38)
+//   4096      230 / 229 (33/31)   251 / 254 (46/48)   314 / 302 (39/31)   338 / 329 (55/48)
+//   6144      254 / 251 (36/45)   273 / 276 (50/57)   343 / 335 (44/46)   369 / 362 (58/58)
+//   8192      269 / 275 (35/38)   290 / 302 (50/59)   369 / 373 (45/38)   401 / 402 (62/59)
+//   10000     286 / 298 (39/41)   312 / 318 (54/60)   400 / 404 (47/40)   426 / 433 (64/62)
+static uint32_t l1_pair_tiles(uint32_t ft_out) { return ft_out < 320 ? 2 * ft_out : 640; }
 
 int32_t launch_ls_l1_forward(const LsDenseArgs& a, hipStream_t stream) {
     TATARA_REQUIRE(a.l1 >= 2 && a.l1 <= 32, "l1 must be in [2, 32]");
@@ -1174,7 +1182,7 @@ int32_t launch_ls_l1_forward(const LsDenseArgs& a, hipStream_t stream) {
             ls_l1_fwd_tf32_kernel<2><<<ceil_div(tiles, 4), 256, 0, stream>>>(a);
         else
             ls_l1_fwd_tf32_kernel<1><<<ceil_div(tiles, 4), 256, 0, stream>>>(a);
-    } else if (tiles < kL1PairTiles) {
+    } else if (tiles < l1_pair_tiles(a.ft_out)) {
         if (two)
             ls_l1_fwd_sums_kernel<2><<<tiles, 256, 0, stream>>>(a);
         else

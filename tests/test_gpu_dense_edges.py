@@ -36,7 +36,9 @@ def test_simple_edges(gpu, ft_out, l1, l2, b):
 
 @pytest.mark.parametrize("ft_out,l1,l2,b,factorize", [(128, 8, 16, 16, True), (384, 16, 32, 48, True),
                                                       (128, 32, 64, 272, False), (640, 32, 16, 1040, True),
-                                                      (128, 16, 64, 34000, False)])
+                                                      (128, 16, 64, 34000, False),
+                                                      # 255 and 256 tiles: the L1 forward's line at 128 columns
+                                                      (128, 32, 16, 3936, False), (128, 32, 16, 3952, False)])
 def test_layerstack_edges(gpu, ft_out, l1, l2, b, factorize):
     sh, cfg = gt.make(ft_out=ft_out, l1=l1, l2=l2, b=b, factorize=factorize)
     batch, bucket = gt.batch_for(b, b, sh.nb)
