@@ -55,6 +55,23 @@ def test_f32_layouts_bit_exact(gpu, b, ft_out, fallback):
         assert np.array_equal(got, want), shift
 
 
+@pytest.mark.parametrize("ft_out", [260, 384, 388])
+def test_padding_of_the_copy_is_not_looked_at(gpu, ft_out):
+    """The chunk-major copy's columns past ft_out hold what an earlier call left:
+    after a call of NaN values the sums are the same bits as after one of zeros
+    (a non-finite value in a row makes the matrix-core form add row by row)."""
+    b, out = 200, []
+    idx = rows(b, False)
+    dft = np.random.default_rng(ft_out).normal(0, 1, (2, b, ft_out)).astype(np.float16).view(np.uint16)
+    for left in (0.0, np.nan):
+        run(gpu, gpu.tatara_op_ft_weight_grad_mfma_f16, np.full((2, b, 508), left, np.float16).view(np.uint16), idx, b,
+            508, 0, 1.0)
+        got, used = run(gpu, gpu.tatara_op_ft_weight_grad_mfma_f16, dft, idx, b, ft_out, 0, 1.0)
+        assert used == 1
+        out.append(got)
+    assert np.array_equal(*out)
+
+
 @pytest.mark.parametrize("b,ft_out", [(1, 256), (66, 512), (130, 260)])
 def test_f16_layouts_agree(gpu, b, ft_out):
     idx = rows(b, False)
